@@ -949,6 +949,146 @@ __global__ __launch_bounds__(NT) void k_ulv_factor(const FInst<T>* __restrict__ 
     for (int e = tid; e < nk; e += blockDim.x) I.fac[f.taulq + e] = taus[e];
 }
 
+// LDS and sizes of the blocked LQ of k_ulv_factor_mf (its comment has the layouts).
+template <typename T>
+struct LqPanel {
+    static constexpr int TPP = 17;
+    static constexpr int pitch(int ntile) { return 16 * ntile + 2; }
+    T *Vs, *Ts, *tl;
+    T* Tg;  // the factor's T blocks (global)
+    int nk, wave, lane;
+};
+
+// Panel P of the blocked LQ and the panels after it: wave P factors its 16 rows, then the
+// waves below apply the block reflector.  P is a template parameter, so every tile loop is
+// straight-line code over the tiles t >= P that still hold columns to reduce.
+//
+// The panel is bound by the serial chain of its 16 reflectors in one wave, so a reflector is
+// one pass: row j (unscaled, masked to its columns right of the diagonal) is put in the
+// panel's V row in LDS and read back by every lane, and one product of it with every row
+// gives row j's own norm (lane j), the dots of the rows below, and the Gram column of the
+// rows above (whose scales their lanes keep).  The scale 1 / (alpha - beta) multiplies the
+// finished dot instead of the vector, so dlarfg's square root and divisions wait for one
+// reduction only and the vector is scaled once, when the panel is done.  T (dlarft forward)
+// is kept in the wave's registers, and reflector j - 1's column of it is formed while row j
+// travels through LDS.  A reflector takes 0.75 us over 64 columns and 1.4 us over 128 (1.6-2.9
+// before); the launches at n = 65536, leaf 128: leaves 848 -> 637 us, levels of 65-128 rows
+// 342 -> 298 us, of up to 64 rows 194 -> 172 us.
+template <typename T, int NTILE, int P>
+__device__ __forceinline__ void lq_panels(typename Mfma<T>::v4 (&a)[NTILE], const LqPanel<T>& L) {
+    using MF = Mfma<T>;
+    using V4 = typename MF::v4;
+    constexpr int NCP = LqPanel<T>::pitch(NTILE), TPP = LqPanel<T>::TPP;
+    const int i0 = 16 * P;
+    if (i0 >= L.nk) return;
+    const int nb = min(16, L.nk - i0), li = L.lane & 15, lk = L.lane >> 4;
+    T* Vp = L.Vs + (P & 1) * 16 * NCP;
+    T* Tp = L.Ts + (P & 1) * 16 * TPP;
+    if (L.wave == P) {
+        T tr[4] = {T(0), T(0), T(0), T(0)};  // T(li, 4 r + lk)
+        T scale = T(0), mytau = T(0);  // of reflector li, once formed
+        T g = T(0), ptau = T(0);       // reflector j - 1's Gram column and tau
+        // T(li, j) = -tau_j sum_{li <= b < j} T(li, b) (v_b . v_j) for li < j (g is zero
+        // from lane j on)
+        auto tcol = [&](int j) {
+            T s = T(0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s += tr[r] * __shfl(g, 4 * r + lk, 64);
+            s = rows_sum(s);
+            const T x = li < j ? -ptau * s : (li == j ? ptau : T(0));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) tr[r] = 4 * r + lk == j ? x : tr[r];
+        };
+        for (int j = 0; j < nb; ++j) {
+            const bool own = li == j;
+            T* vrow = Vp + j * NCP;  // slot 16 t + 4 lk + r: a lane's 4 values of a tile
+            T aj = T(0);
+            if (own) {
+                V4 v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = MF::row(lk, r) > j ? a[P][r] : T(0);
+                *reinterpret_cast<V4*>(vrow + 16 * P + 4 * lk) = v;
+#pragma unroll
+                for (int t = P + 1; t < NTILE; ++t) *reinterpret_cast<V4*>(vrow + 16 * t + 4 * lk) = a[t];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int r = 0; r < 4; ++r) aj += MF::row(lk, r) == j ? a[P][r] : T(0);
+            aj = rows_sum(aj);
+            if (j > 0) tcol(j - 1);
+            V4 d4 = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+            for (int t = P; t < NTILE; ++t) {
+                const V4 v = *reinterpret_cast<const V4*>(vrow + 16 * t + 4 * lk);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) d4[r] += a[t][r] * v[r];
+            }
+            T d = rows_sum((d4[0] + d4[1]) + (d4[2] + d4[3]));
+            T beta, tau, scl;
+            larfg(lane_read(aj, j), lane_read(d, j), beta, tau, scl);
+            d = aj + scl * d;  // v_j . row li
+            const T dt = li > j ? tau * d : T(0);
+            const T ds = dt * scl;
+            // more than four tiles: read the vector again rather than keep it (the rows
+            // already hold 4 NTILE values a lane)
+            if (NTILE - P > 4) asm volatile("" ::: "memory");
+#pragma unroll
+            for (int t = P; t < NTILE; ++t) {
+                const V4 v = *reinterpret_cast<const V4*>(vrow + 16 * t + 4 * lk);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[t][r] -= ds * v[r];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (MF::row(lk, r) == j) a[P][r] = own ? beta : a[P][r] - dt;
+            g = li < j ? scale * d : T(0);
+            ptau = tau;
+            scale = own ? scl : scale;
+            mytau = own ? tau : mytau;
+        }
+        tcol(nb - 1);
+        // the reflectors scaled, in the rows and (columns in order, rows beyond nb zero) in
+        // LDS; T to LDS and to the factor (rows and columns beyond nb zero)
+#pragma unroll
+        for (int t = P; t < NTILE; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int cr = 16 * (t - P) + MF::row(lk, r);  // column of the panel
+                const T x = a[t][r] * scale;
+                if (li < nb && cr > li) a[t][r] = x;
+                Vp[li * NCP + 16 * P + cr] = li < nb ? (cr < li ? T(0) : (cr == li ? T(1) : x)) : T(0);
+            }
+        T* Tg = L.Tg + (int64_t)P * NB * NB;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const T x = li < nb ? tr[r] : T(0);
+            Tp[li * TPP + 4 * r + lk] = x;
+            Tg[li + (4 * r + lk) * NB] = x;
+        }
+        if (lk == 0 && li < nb) L.tl[i0 + li] = mytau;
+    }
+    __syncthreads();
+    if (L.wave > P) {
+        // W <- W - ((W V') T) V for this wave's rows, as Wt -= V' (T' (V Wt)); V is zero left
+        // of tile P
+        V4 Pw = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+        for (int t = P; t < NTILE; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) Pw = MF::mac(Vp[li * NCP + 16 * t + MF::row(lk, r)], a[t][r], Pw);
+        V4 Q = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Q = MF::mac(Tp[MF::row(lk, r) * TPP + li], Pw[r], Q);
+#pragma unroll
+        for (int t = P; t < NTILE; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) a[t] = MF::mac(-Vp[MF::row(lk, r) * NCP + 16 * t + li], Q[r], a[t]);
+    }
+    if constexpr (P + 1 < NTILE) lq_panels<T, NTILE, P + 1>(a, L);
+}
+
 // Blocked factor of one node per workgroup, on MFMA (NT threads, 16 rows of W = [D; V']
 // per wave, n <= 16 NTILE).  Phases 0-2 as ulv_front.  Then each wave keeps its 16 rows of W
 // in registers, transposed, in the accumulator layout of the 16x16x4 MFMA: lane l holds row
@@ -1020,161 +1160,14 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
     // [2][16][NCP]: the panel's reflectors (row-major).  The row pitch NC + 2 doubles puts the
     // 16 rows a column read touches (lanes li) in distinct LDS banks (a pitch of NC = 64 or
     // 128 maps them all to one) and keeps every row 16-byte aligned for the vector reads.
-    constexpr int NCP = NC + 2;
+    constexpr int NCP = LqPanel<T>::pitch(NTILE);
     T* Vs = reinterpret_cast<T*>(lds_raw);
     // [2][16][TPP]: T(a, q) at a * TPP + q; the pitch 17 puts the 16 rows (lanes li) in
     // distinct LDS banks
-    constexpr int TPP = 17;
+    constexpr int TPP = LqPanel<T>::TPP;
     T* Ts = Vs + 2 * 16 * NCP;
     T* tl = Ts + 2 * 16 * TPP;              // nk taus (nk <= n <= 128)
-    T* Gs = tl + 128;                       // [16]: the panel step's Gram column v_b . v_j
-    const int npan = (nk + 15) / 16;
-    for (int p = 0; p < npan; ++p) {
-        const int i0 = 16 * p, nb = min(16, nk - i0), buf = p & 1;
-        T* Vp = Vs + buf * 16 * NCP;
-        T* Tp = Ts + buf * 16 * TPP;
-        if (wave == p) {
-            // the panel's reflectors, one row at a time (a loop, not unrolled), each applied
-            // to the wave's later rows.  Rows live in the 4 lanes l%16 of the wave's 16-lane
-            // rows, so a row's sums are rows_sum; row j's norm and pivot reach every lane by
-            // readlane, and its reflector v_j reaches the other rows through row j of the
-            // panel's V buffer in LDS (written by row j's lanes, read back by every lane; one
-            // wave, so LDS order is program order).  Columns left of the panel (tiles t < p)
-            // are already reduced and skipped.  The same dot loop gives v_b . v_j for the
-            // panel's earlier reflectors b < j (their masked rows), which builds column j of
-            // T (dlarft forward) through the 16-entry Gram column Gs.  Row ra of T lives in
-            // LDS (Tp[ra * TPP + q]); the 4 lanes of row ra write the same values.
-            const int ra = li;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) Tp[ra * TPP + q] = T(0);
-            // Only tile p (the panel's own 16 columns) needs column masks; in tiles t > p every
-            // column is right of the reflector (c > i) and of every panel row's diagonal.  In
-            // tile p, column 16 p + cr with cr = Mfma<T>::row(lk, r).  Row j's reflector is
-            // stored lane-contiguously (slot 16 t + 4 lk + r) so each lane reads its 4 values
-            // of a tile as one vector.
-            for (int j = 0; j < nb; ++j) {
-                const int i = i0 + j;
-                T part = T(0), al = T(0);
-#pragma unroll
-                for (int t = 0; t < NTILE; ++t) {
-                    if (t < p) continue;
-                    if (t == p) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int cr = MF::row(lk, r);
-                            const T x = a[t][r];
-                            part += cr > j ? x * x : T(0);
-                            al += cr == j ? x : T(0);
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) part += a[t][r] * a[t][r];
-                    }
-                }
-                const T xn2 = lane_read(rows_sum(part), j);
-                const T alpha = lane_read(rows_sum(al), j);
-                T beta, tau, scl;
-                larfg(alpha, xn2, beta, tau, scl);
-                // row j becomes [L, beta, v_j]; its lanes also store v_j = [0, 1, x scl]
-                const bool own = li == j;
-                T* vrow = Vp + j * NCP;
-#pragma unroll
-                for (int t = 0; t < NTILE; ++t) {
-                    if (t < p) continue;
-                    V4 v;
-                    if (t == p) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int cr = MF::row(lk, r);
-                            const T x = a[t][r];
-                            v[r] = cr > j ? x * scl : (cr == j ? T(1) : T(0));
-                            a[t][r] = own ? (cr == j ? beta : (cr > j ? v[r] : x)) : x;
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            v[r] = a[t][r] * scl;
-                            a[t][r] = own ? v[r] : a[t][r];
-                        }
-                    }
-                    if (own) *reinterpret_cast<V4*>(vrow + 16 * t + 4 * lk) = v;
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                // d = row . v_j for the rows below j; v_li . v_j for the reflectors above
-                // (row li < j reads as [0, 1, v] about its diagonal column 16 p + li)
-                T d = T(0);
-#pragma unroll
-                for (int t = 0; t < NTILE; ++t) {
-                    if (t < p) continue;
-                    const V4 v = *reinterpret_cast<const V4*>(vrow + 16 * t + 4 * lk);
-                    if (t == p) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int cr = MF::row(lk, r);
-                            const T x = a[t][r];
-                            const T left = li > j ? x : (cr < li ? T(0) : (cr == li ? T(1) : x));
-                            d += left * v[r];
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) d += a[t][r] * v[r];
-                    }
-                }
-                d = rows_sum(d);
-                const T dt = li > j ? d * tau : T(0);
-#pragma unroll
-                for (int t = 0; t < NTILE; ++t) {
-                    if (t < p) continue;
-                    const V4 v = *reinterpret_cast<const V4*>(vrow + 16 * t + 4 * lk);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) a[t][r] -= dt * v[r];
-                }
-                // T(a, j) = -tau_j sum_{a <= b < j} T(a, b) (v_b . v_j) for a < j
-                Gs[li] = d;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                T acc = T(0);
-                for (int b2 = 0; b2 < j; ++b2) acc += Tp[ra * TPP + b2] * Gs[b2];
-                Tp[ra * TPP + j] = ra < j ? -tau * acc : (ra == j ? tau : T(0));
-                if (lane == 0) tl[i] = tau;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            }
-            // V (rows beyond nb zero) and T to LDS; T also to the factor
-#pragma unroll
-            for (int t = 0; t < NTILE; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int c = colof(t, r), ii = i0 + li;
-                    Vp[li * NCP + c] = li < nb ? (c < ii ? T(0) : (c == ii ? T(1) : a[t][r])) : T(0);
-                }
-            if (lane < 16) {
-                T* Tg = I.fac + f.Tlq + (int64_t)p * NB * NB;
-#pragma unroll
-                for (int q = 0; q < 16; ++q) Tg[ra + q * NB] = (q < nb && ra < nb) ? Tp[ra * TPP + q] : T(0);
-            }
-        }
-        __syncthreads();
-        if (wave > p) {
-            // W <- W - ((W V') T) V for this wave's rows, as Wt -= V' (T' (V Wt))
-            V4 P = {T(0), T(0), T(0), T(0)};
-#pragma unroll
-            for (int t = 0; t < NTILE; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) P = MF::mac(Vp[li * NCP + colof(t, r)], a[t][r], P);
-            V4 Q = {T(0), T(0), T(0), T(0)};
-#pragma unroll
-            for (int r = 0; r < 4; ++r) Q = MF::mac(Tp[MF::row(lk, r) * TPP + li], P[r], Q);
-#pragma unroll
-            for (int t = 0; t < NTILE; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) a[t] = MF::mac(-Vp[MF::row(lk, r) * NCP + 16 * t + li], Q[r], a[t]);
-        }
-    }
+    lq_panels<T, NTILE, 0>(a, LqPanel<T>{Vs, Ts, tl, I.fac + f.Tlq, nk, wave, lane});
     __syncthreads();
 
     // ---- outputs (the same blocks and layouts as k_ulv_factor's phase 5) ----
@@ -2756,7 +2749,7 @@ static hipError_t launch_factor_mf_tile(const FInst<T>* insts, const WorkItem* w
                                         hipStream_t st) {
     if (waves <= 8) return launch_factor_mf_nt<T, NTILE, 512>(insts, work, nwork, lds, st);
     if (waves <= 12) return launch_factor_mf_nt<T, NTILE, 768>(insts, work, nwork, lds, st);
-    if (sizeof(T) == 4) return launch_factor_mf_nt<T, NTILE, 1024>(insts, work, nwork, lds, st);
+    if constexpr (sizeof(T) == 4) return launch_factor_mf_nt<T, NTILE, 1024>(insts, work, nwork, lds, st);
     return hipErrorInvalidValue;
 }
 int factor_mf_max_rows(int elem_bytes) { return elem_bytes == 8 ? 192 : 256; }
