@@ -2674,21 +2674,31 @@ __global__ void k_colnorm2(const double* __restrict__ A, int64_t lda, int64_t n,
     }
 }
 
-// Batched refinement helpers: block (request, column).
-// r = b - r (r holds A x on entry); norms[2*(req*maxc + col)] = ||b||^2, [+1] = ||r||^2
-__global__ void k_resid_batch(const BatchVec* __restrict__ tab, int maxc, double* __restrict__ norms) {
-    const BatchVec v = tab[blockIdx.x];
-    const int j = blockIdx.y;
-    if (j >= v.nrhs) return;
+// r = b - r (r holds A x on entry) with both squared column norms from the same pass: thread
+// t of a workgroup of NT takes rows i0 + t + q NT of [i0, i1), U of them in flight at once.
+// The result is valid in thread 0.
+template <int NT, int U>
+__device__ __forceinline__ void resid_norms(const double* __restrict__ b, double* __restrict__ r, int64_t i0, int64_t i1,
+                                            double& nb, double& nr) {
     double sb = 0.0, sr = 0.0;
-    for (int64_t i = threadIdx.x; i < v.n; i += blockDim.x) {
-        const double bi = v.b[i + j * v.ldb];
-        const double ri = bi - v.r[i + j * v.n];
-        v.r[i + j * v.n] = ri;
-        sb += bi * bi;
-        sr += ri * ri;
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += U * NT) {
+        double bv[U], rv[U];
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const int64_t e = i + q * NT;
+            bv[q] = e < i1 ? b[e] : 0.0;
+            rv[q] = e < i1 ? r[e] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const int64_t e = i + q * NT;
+            const double d = bv[q] - rv[q];
+            if (e < i1) r[e] = d;
+            sb += bv[q] * bv[q];
+            sr += d * d;
+        }
     }
-    __shared__ double red[2][16];
+    __shared__ double red[2][NT / 64];
     sb = wave_reduce(sb);
     sr = wave_reduce(sr);
     if ((threadIdx.x & 63) == 0) {
@@ -2696,23 +2706,68 @@ __global__ void k_resid_batch(const BatchVec* __restrict__ tab, int maxc, double
         red[1][threadIdx.x >> 6] = sr;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double tb = 0.0, trr = 0.0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-            tb += red[0][w];
-            trr += red[1][w];
+    nb = nr = 0.0;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < NT / 64; ++w) {
+            nb += red[0][w];
+            nr += red[1][w];
         }
-        norms[2 * ((int64_t)blockIdx.x * maxc + j)] = tb;
-        norms[2 * ((int64_t)blockIdx.x * maxc + j) + 1] = trr;
+}
+
+// Residual of one solve, block (column, chunk of RESID_ROWS rows): out[2 (chunk nrhs + j)] =
+// the chunk's share of ||b_j||^2, [+1] of ||r_j||^2; the host adds the chunks in order.
+// Bound by memory: two reads and a write.  One workgroup a column (as one norm of it was
+// before) is bound by latency instead, 64 us a norm of 65536 x 128; with 16 rows a thread in
+// flight and 16 x 128 workgroups the whole pass takes 32 us (residual and two norms: 160).
+__global__ __launch_bounds__(256) void k_resid_norms(const double* __restrict__ B, int64_t ldb, double* __restrict__ Rr,
+                                                     int64_t ldr, int64_t n, int nrhs, double* __restrict__ out) {
+    const int j = blockIdx.x;
+    const int64_t i0 = (int64_t)blockIdx.y * RESID_ROWS;
+    double nb, nr;
+    resid_norms<256, 8>(B + j * ldb, Rr + j * ldr, i0, min(n, i0 + RESID_ROWS), nb, nr);
+    if (threadIdx.x == 0) {
+        out[2 * ((int64_t)blockIdx.y * nrhs + j)] = nb;
+        out[2 * ((int64_t)blockIdx.y * nrhs + j) + 1] = nr;
     }
 }
 
-// x += d for active requests
-__global__ void k_axpy_batch(const BatchVec* __restrict__ tab) {
+// Batched refinement helpers: block (request, column).
+// r = b - r (r holds A x on entry); norms[2*(req*maxc + col)] = ||b||^2, [+1] = ||r||^2.
+// Latency-bound where requests are few: 1024 threads with four rows each in flight take a
+// 32768-row column in 8 rounds (256 threads, one row at a time, were 128 rounds and 64 us
+// for 16 requests of up to 32 columns; now 32 us).
+__global__ __launch_bounds__(1024) void k_resid_batch(const BatchVec* __restrict__ tab, int maxc, double* __restrict__ norms) {
     const BatchVec v = tab[blockIdx.x];
     const int j = blockIdx.y;
     if (j >= v.nrhs) return;
-    for (int64_t i = threadIdx.x; i < v.n; i += blockDim.x) v.x[i + j * v.ldx] += v.d[i + j * v.n];
+    double nb, nr;
+    resid_norms<1024, 4>(v.b + j * v.ldb, v.r + j * v.n, 0, v.n, nb, nr);
+    if (threadIdx.x == 0) {
+        norms[2 * ((int64_t)blockIdx.x * maxc + j)] = nb;
+        norms[2 * ((int64_t)blockIdx.x * maxc + j) + 1] = nr;
+    }
+}
+
+// x += d for active requests, block (request, column), 1024 threads with four rows each in
+// flight as above (38 -> 19 us)
+__global__ __launch_bounds__(1024) void k_axpy_batch(const BatchVec* __restrict__ tab) {
+    const BatchVec v = tab[blockIdx.x];
+    const int j = blockIdx.y;
+    if (j >= v.nrhs) return;
+    double* __restrict__ x = v.x + j * v.ldx;
+    const double* __restrict__ d = v.d + j * v.n;
+    for (int64_t i = threadIdx.x; i < v.n; i += 4 * 1024) {
+        double xv[4], dv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t e = i + q * 1024;
+            xv[q] = e < v.n ? x[e] : 0.0;
+            dv[q] = e < v.n ? d[e] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (i + q * 1024 < v.n) x[i + q * 1024] = xv[q] + dv[q];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2996,12 +3051,12 @@ hipError_t launch_refine_check(BatchVec* tab, char* sinst0, char* sinst1, int64_
 }
 hipError_t launch_resid_batch(const BatchVec* tab, int cnt, int maxc, double* norms, hipStream_t st) {
     if (cnt <= 0 || maxc <= 0) return hipSuccess;
-    klaunch(k_resid_batch, dim3(cnt, maxc), dim3(256), 0, st, tab, maxc, norms);
+    klaunch(k_resid_batch, dim3(cnt, maxc), dim3(1024), 0, st, tab, maxc, norms);
     return hipGetLastError();
 }
 hipError_t launch_axpy_batch(const BatchVec* tab, int cnt, int maxc, hipStream_t st) {
     if (cnt <= 0 || maxc <= 0) return hipSuccess;
-    klaunch(k_axpy_batch, dim3(cnt, maxc), dim3(256), 0, st, tab);
+    klaunch(k_axpy_batch, dim3(cnt, maxc), dim3(1024), 0, st, tab);
     return hipGetLastError();
 }
 
@@ -3140,6 +3195,14 @@ hipError_t launch_residual(const double* B, int64_t ldb, double* R, int64_t ldr,
     if (blocks > 4096) blocks = 4096;
     if (blocks < 1) return hipSuccess;
     klaunch(k_residual, dim3(blocks), dim3(256), 0, st, B, ldb, R, ldr, n, nrhs);
+    return hipGetLastError();
+}
+hipError_t launch_resid_norms(const double* B, int64_t ldb, double* R, int64_t ldr, int64_t n, int nrhs, double* out,
+                              hipStream_t st) {
+    if (n <= 0 || nrhs <= 0) return hipSuccess;
+    const int64_t chunks = (n + RESID_ROWS - 1) / RESID_ROWS;
+    if (chunks > 65535) return hipErrorInvalidValue;
+    klaunch(k_resid_norms, dim3(nrhs, (unsigned)chunks), dim3(256), 0, st, B, ldb, R, ldr, n, nrhs, out);
     return hipGetLastError();
 }
 hipError_t launch_axpy(double* X, int64_t ldx, const double* D, int64_t ldd, int64_t n, int nrhs, hipStream_t st) {

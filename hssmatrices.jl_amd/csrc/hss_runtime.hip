@@ -2425,6 +2425,8 @@ static hss_status solve_one(hss_fact_s* F, int nrhs, const double* dB, int64_t l
                                F->lds_groot_res, F->lds_groot2, F->lds_groot2s, st);
 }
 
+static size_t resid_chunks(int64_t n) { return (size_t)((std::max<int64_t>(n, 1) + RESID_ROWS - 1) / RESID_ROWS); }
+
 static hss_status ensure_refine(hss_fact_s* F, int nrhs) {
     const size_t need = (size_t)std::max<int64_t>(F->mat->rows, 1) * nrhs;
     if (need <= F->rf_cap) return HSS_OK;
@@ -2435,23 +2437,25 @@ static hss_status ensure_refine(hss_fact_s* F, int nrhs) {
     F->rf_cap = 0;
     HIP_TRY(dalloc(&F->d_r, need));
     HIP_TRY(dalloc(&F->d_d, need));
-    HIP_TRY(dalloc(&F->d_nrm, (size_t)2 * nrhs));
+    HIP_TRY(dalloc(&F->d_nrm, 2 * (size_t)nrhs * resid_chunks(F->mat->rows)));
     F->rf_cap = need;
     return HSS_OK;
 }
 
-// max_j ||r_j|| / ||b_j||
-static hss_status rel_residual(hss_fact_s* F, int nrhs, const double* dB, int64_t ldb, const double* dR, int64_t ldr,
-                               hipStream_t st, double* out) {
+// R = B - R (R holds A X on entry); *out = max_j ||r_j|| / ||b_j||
+static hss_status residual_norm(hss_fact_s* F, int nrhs, const double* dB, int64_t ldb, double* dR, int64_t ldr,
+                                hipStream_t st, double* out) {
     const int64_t n = F->mat->rows;
-    HIP_TRY(launch_colnorm2(dB, ldb, n, nrhs, F->d_nrm, st));
-    HIP_TRY(launch_colnorm2(dR, ldr, n, nrhs, F->d_nrm + nrhs, st));
-    std::vector<double> h(2 * (size_t)nrhs);
-    HIP_TRY(hipMemcpyAsync(h.data(), F->d_nrm, sizeof(double) * 2 * nrhs, hipMemcpyDeviceToHost, st));
+    HIP_TRY(launch_resid_norms(dB, ldb, dR, ldr, n, nrhs, F->d_nrm, st));
+    const size_t chunks = resid_chunks(n);
+    std::vector<double> h(2 * (size_t)nrhs * chunks);
+    HIP_TRY(hipMemcpyAsync(h.data(), F->d_nrm, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
+    for (size_t c = 1; c < chunks; ++c)
+        for (size_t e = 0; e < 2 * (size_t)nrhs; ++e) h[e] += h[c * 2 * nrhs + e];
     double worst = 0.0;
     for (int j = 0; j < nrhs; ++j) {
-        const double nb = std::sqrt(h[j]), nr = std::sqrt(h[nrhs + j]);
+        const double nb = std::sqrt(h[2 * j]), nr = std::sqrt(h[2 * j + 1]);
         const double rel = nb > 0 ? nr / nb : nr;
         worst = std::max(worst, rel);
     }
@@ -2629,8 +2633,7 @@ static hss_status solve_dev_impl(hss_fact_s* F, int nrhs, const double* dB, int6
             // r = b - A x   (Float64 HSS matvec)
             s = matmul_enqueue(M, nrhs, 1.0, dX, ldx, 0.0, F->d_r, n);
             if (s != HSS_OK) return s;
-            HIP_TRY(launch_residual(dB, ldb, F->d_r, n, n, nrhs, st));
-            s = rel_residual(F, nrhs, dB, ldb, F->d_r, n, st, &rel);
+            s = residual_norm(F, nrhs, dB, ldb, F->d_r, n, st, &rel);
             if (s != HSS_OK) return s;
             if (rel <= o.tol || it >= o.max_iter) break;
             // d = A \ r with the resident factor (mode 1) or by GMRES preconditioned with it
