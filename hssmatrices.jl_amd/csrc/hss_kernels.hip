@@ -12,7 +12,7 @@
 //   k_ulv_factor  per node: merge of the children (ulvfactor.jl:74-79), QL of U,
 //                 Q'D, LQ of the top rows with the reflectors applied to the
 //                 bottom rows and to V' (ulvfactor.jl:39-54)
-//   k_ulv_wy      compact-WY blocks of the LQ reflectors
+//   k_ulv_wy      compact-WY blocks of the LQ reflectors (k_ulv_factor_mf forms its own)
 //   k_ulv_root    merge + LU with partial pivoting of the root block (ulvfactor.jl:82-86)
 //   k_ulv_rinv    the root block's inverse and merge operator
 //   k_ulv_gform / k_ulv_qform   explicit per-node solve operators (Gz, Gr, Qt), formed
@@ -366,6 +366,9 @@ struct Mfma<double> {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
     static __device__ __forceinline__ int row(int lk, int r) { return 4 * r + lk; }
+    // the l/16 and the register of row q
+    static constexpr int lane_of(int q) { return q & 3; }
+    static constexpr int reg_of(int q) { return q >> 2; }
 };
 template <>
 struct Mfma<float> {
@@ -374,6 +377,8 @@ struct Mfma<float> {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
     static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
+    static constexpr int lane_of(int q) { return q >> 2; }
+    static constexpr int reg_of(int q) { return q & 3; }
 };
 
 // ---------------------------------------------------------------------------
@@ -1103,7 +1108,7 @@ __device__ __forceinline__ void lq_panels(typename Mfma<T>::v4 (&a)[NTILE], cons
 //   below applies the block, W <- W (I - V' T V) = W - ((W V') T) V, as three MFMA chains.
 //   One workgroup barrier per panel (V and T double-buffered).
 // Outputs as k_ulv_factor (L1, the LQ reflectors, L2a, V_top, the reduced D and V, taus)
-// plus the T blocks.
+// plus the T blocks and the inverted diagonal blocks of L1 (k_ulv_wy's outputs).
 template <typename T, int NTILE, int NT>
 __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict__ insts,
                                                       const WorkItem* __restrict__ work, int64_t lds_elems) {
@@ -1168,6 +1173,30 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
     T* Ts = Vs + 2 * 16 * NCP;
     T* tl = Ts + 2 * 16 * TPP;              // nk taus (nk <= n <= 128)
     lq_panels<T, NTILE, 0>(a, LqPanel<T>{Vs, Ts, tl, I.fac + f.Tlq, nk, wave, lane});
+    // Inverse of L1's diagonal block `wave`, which this wave holds: lane li solves L x = e_li.
+    // (A kernel of its own after the factor, which also formed T again, took 245 us on 1022
+    // nodes, one wave a block and its operands from memory.)
+    if (16 * wave < nk) {
+        const int nb = min(16, nk - 16 * wave);
+        V4 d = a[0];
+#pragma unroll
+        for (int t = 1; t < NTILE; ++t)
+            if (wave == t) d = a[t];
+        T x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            T s = i == li ? T(1) : T(0);
+#pragma unroll
+            for (int q = 0; q < i; ++q) s -= lane_read(d[MF::reg_of(q)], 16 * MF::lane_of(q) + i) * x[q];
+            const T dii = lane_read(d[MF::reg_of(i)], 16 * MF::lane_of(i) + i);
+            x[i] = i < nb && li < nb ? s / dii : T(0);
+        }
+        T* Lig = I.fac + f.L1inv + (int64_t)wave * NB * NB;
+        if (lk == 0) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) Lig[q + li * NB] = x[q];
+        }
+    }
     __syncthreads();
 
     // ---- outputs (the same blocks and layouts as k_ulv_factor's phase 5) ----
@@ -1203,7 +1232,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
 
 // Compact-WY T blocks of the LQ reflectors (dlarft, forward columnwise) and the
 // inverted diagonal blocks of L1, from the factor data in global memory: one
-// wave per block of NB reflectors.
+// wave per block of NB reflectors.  For the nodes of k_ulv_factor.
 template <typename T>
 __global__ __launch_bounds__(256) void k_ulv_wy(const FInst<T>* __restrict__ insts, const WorkItem* __restrict__ work) {
     const WorkItem wi = work[blockIdx.x];
@@ -1555,6 +1584,209 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_ulv_qform(const FInst<TF>* __
         __syncthreads();
     }
     unstage(I.fac + f.Qt + (int64_t)j0 * n, n, z, 0, n, nt);
+}
+
+// acc += op(A)(i0 + li, k0 + .) x over the 16 rows of one accumulator-layout tile x (rows
+// k0 .. k0 + 15 of a 16-column block), masked to M x K; A column-major, op = ' when TA.
+// The accumulator layout is the B operand's, so a product's result feeds the next one from
+// its registers.
+template <bool TA, typename TF>
+__device__ __forceinline__ typename Mfma<TF>::v4 tile_mac(const TF* __restrict__ A, int64_t lda, int i0, int M, int k0, int K,
+                                                          typename Mfma<TF>::v4 x, typename Mfma<TF>::v4 acc, int li, int lk,
+                                                          bool neg) {
+    const int i = i0 + li;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int kk = k0 + Mfma<TF>::row(lk, r);
+        TF v = TF(0);
+        if (i < M && kk < K) v = TA ? A[kk + (int64_t)i * lda] : A[i + (int64_t)kk * lda];
+        acc = Mfma<TF>::mac(neg ? -v : v, x[r], acc);
+    }
+    return acc;
+}
+
+// k_ulv_gform and k_ulv_qform for nodes of at most 16 NTILE rows: a wave forms 16 columns of
+// the operator by itself, the column's rows in registers (accumulator layout), every product
+// one MFMA chain with the factor block streamed from memory, no LDS and no barrier.  Unit
+// input columns need no product for the children's merge, the u part and (leaves) Y' b: they
+// are columns of P12 / P21, rows of W and rows of Y.  Bound by the MFMA chain of one wave
+// (about 360 MFMAs, 64 cycles each, for a 128-row leaf).  The LDS kernels run one or two of a
+// workgroup's four waves on the 16-row blocks, with two barriers a block.
+// n = 65536, leaf 128 (1022 nodes): Gz and Gr 370 -> 233 us, Qt 163 -> 143; 32 Cauchy matrices
+// of leaf 64: 961 -> 349 and 187 -> 151 us.
+template <typename TF, int NTILE>
+__global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_gform_w(const FInst<TF>* __restrict__ insts,
+                                                                         const WorkItem* __restrict__ work) {
+    using MF = Mfma<TF>;
+    using V4 = typename MF::v4;
+    const WorkItem wi = work[blockIdx.x];
+    const FInst<TF>& I = insts[wi.inst];
+    const DevNode nd = I.nodes[wi.node];
+    const FNode f = I.fn[wi.node];
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int j0 = 16 * (blockIdx.y * 4 + (threadIdx.x >> 6));
+    const int Kx = f.Kx, nk = f.nk, mr = f.mr, kv = nd.kv, R = mr + kv, m = f.m, k = f.k;
+    if (j0 >= Kx + nk) return;
+    TF* Gr = I.fac + f.Gr;  // ld R
+    // columns [Kx, Kx + nk) of Gr: [-L2a; V_top']
+    for (int c = max(j0, Kx); c < min(j0 + 16, Kx + nk); ++c) {
+        const int l = c - Kx;
+        for (int i = lane; i < R; i += 64)
+            Gr[i + (int64_t)c * R] = i < mr ? -I.fac[f.L2a + i + (int64_t)l * k] : I.fac[f.Vt + l + (int64_t)(i - mr) * nk];
+    }
+    if (j0 >= Kx) return;
+    const int c = j0 + li;  // this lane's input column
+    const bool on = c < Kx;
+    // b for x = e_c: a unit row, or (u_1, u_2) a column of -P21 or -P12 over rows [p0, p1);
+    // (ulvfactor.jl:74: b = [b_1 - P12 u_2; b_2 - P21 u_1])
+    int unit = on && nd.is_leaf ? c : -1, p0 = 0, p1 = 0, wl = 0;
+    const TF* pc = I.fac;
+    const double* wc = nullptr;  // W' e_l is row l of W (wl rows)
+    if (on && !nd.is_leaf) {
+        const DevNode dl = I.nodes[nd.left], dr = I.nodes[nd.right];
+        const int mrl = I.fn[nd.left].mr;
+        if (c < mrl) unit = c;
+        else if (c < mrl + dl.kv) {
+            pc = I.fac + f.P21 + (int64_t)(c - mrl) * (m - mrl);
+            p0 = mrl;
+            p1 = m;
+            wc = I.blob + dl.W + (c - mrl);
+            wl = dl.kv;
+        } else if (c < m + dl.kv) unit = c - dl.kv;
+        else {
+            pc = I.fac + f.P12 + (int64_t)(c - m - dl.kv) * mrl;
+            p1 = mrl;
+            wc = I.blob + dr.W + (c - m - dl.kv);
+            wl = dr.kv;
+        }
+    }
+    V4 b[NTILE];
+#pragma unroll
+    for (int t = 0; t < NTILE; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * t + MF::row(lk, r);
+            TF v = row == unit ? TF(1) : TF(0);
+            if (row >= p0 && row < p1) v = -pc[row - p0];
+            b[t][r] = v;
+        }
+    if (!f.pass && k > 0) {
+        // b <- Q_ql' b = b - Y (T (Y' b))   (ulvfactor.jl:42)
+        const TF* Y = I.fac + f.Yql;
+        const TF* Tq = I.fac + f.Tql;
+        V4 t1[NTILE];
+#pragma unroll
+        for (int q = 0; q < NTILE; ++q) {
+            t1[q] = V4{TF(0), TF(0), TF(0), TF(0)};
+            if (16 * q >= k) continue;
+            if (nd.is_leaf) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int kk = 16 * q + MF::row(lk, r);
+                    if (on && kk < k) t1[q][r] = Y[c + (int64_t)kk * m];
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < NTILE; ++t) t1[q] = tile_mac<true, TF>(Y, m, 16 * q, k, 16 * t, m, b[t], t1[q], li, lk, false);
+            }
+        }
+        // T is upper triangular: rows of tile q take tiles q and right of it, so t1 is
+        // overwritten from the top
+#pragma unroll
+        for (int q = 0; q < NTILE; ++q) {
+            if (16 * q >= k) continue;
+            V4 s = {TF(0), TF(0), TF(0), TF(0)};
+#pragma unroll
+            for (int t = q; t < NTILE; ++t)
+                if (16 * t < k) s = tile_mac<false, TF>(Tq, k, 16 * q, k, 16 * t, k, t1[t], s, li, lk, false);
+            t1[q] = s;
+        }
+#pragma unroll
+        for (int q = 0; q < NTILE; ++q) {
+            if (16 * q >= k) continue;
+#pragma unroll
+            for (int t = 0; t < NTILE; ++t) b[t] = tile_mac<false, TF>(Y, m, 16 * t, m, 16 * q, k, t1[q], b[t], li, lk, true);
+        }
+    }
+    // reduced b: (Q_ql' b)[nk:m] (all of b where nothing is eliminated)
+    if (on) {
+#pragma unroll
+        for (int t = 0; t < NTILE; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * t + MF::row(lk, r);
+                if (row >= nk && row < m) Gr[row - nk + (int64_t)c * R] = b[t][r];
+            }
+        // u part: W_1' u_1 + W_2' u_2 (ulvfactor.jl:89)
+        for (int i = lk; i < kv; i += 4) Gr[mr + i + (int64_t)c * R] = wc ? (TF)wc[(int64_t)i * wl] : TF(0);
+    }
+    // zloc = L1 \ b[0:nk]  (ulvfactor.jl:48), blocked with inverted diagonal blocks (whose
+    // columns beyond nk are zero); zloc replaces b tile by tile
+    const TF* L1 = I.fac + f.L1;
+#pragma unroll
+    for (int q = 0; q < NTILE; ++q) {
+        if (16 * q >= nk) continue;
+        V4 s = b[q];
+#pragma unroll
+        for (int t = 0; t < q; ++t) s = tile_mac<false, TF>(L1, nk, 16 * q, nk, 16 * t, nk, b[t], s, li, lk, true);
+        b[q] = tile_mac<false, TF>(I.fac + f.L1inv + (int64_t)q * NB * NB, NB, 0, NB, 0, NB, s, V4{TF(0), TF(0), TF(0), TF(0)},
+                                   li, lk, false);
+    }
+    if (on) {
+        TF* Gz = I.fac + f.Gz + (int64_t)c * nk;
+#pragma unroll
+        for (int t = 0; t < NTILE; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * t + MF::row(lk, r);
+                if (row < nk) Gz[row] = b[t][r];
+            }
+    }
+}
+
+// Qt as k_ulv_qform forms it, 16 columns a wave (see k_ulv_gform_w).  A block of reflectors
+// below a column's unit row leaves it alone, so the wave starts at its own tile's block.
+template <typename TF, int NTILE>
+__global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_qform_w(const FInst<TF>* __restrict__ insts,
+                                                                         const WorkItem* __restrict__ work) {
+    using MF = Mfma<TF>;
+    using V4 = typename MF::v4;
+    const WorkItem wi = work[blockIdx.x];
+    const FInst<TF>& I = insts[wi.inst];
+    const FNode f = I.fn[wi.node];
+    if (f.Qt < 0) return;
+    const int n = f.n, nk = f.nk;
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int j0 = 16 * (blockIdx.y * 4 + (threadIdx.x >> 6));
+    if (j0 >= n) return;
+    const int c = j0 + li;
+    V4 z[NTILE];
+#pragma unroll
+    for (int t = 0; t < NTILE; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[t][r] = 16 * t + MF::row(lk, r) == c ? TF(1) : TF(0);
+    const TF* Y = I.fac + f.Ylq;
+#pragma unroll
+    for (int q = NTILE - 1; q >= 0; --q) {
+        if (16 * q >= nk || 16 * q > j0) continue;
+        V4 t1 = {TF(0), TF(0), TF(0), TF(0)};
+#pragma unroll
+        for (int t = q; t < NTILE; ++t) t1 = tile_mac<true, TF>(Y, n, 16 * q, nk, 16 * t, n, z[t], t1, li, lk, false);
+        t1 = tile_mac<false, TF>(I.fac + f.Tlq + (int64_t)q * NB * NB, NB, 0, NB, 0, NB, t1, V4{TF(0), TF(0), TF(0), TF(0)}, li,
+                                 lk, false);
+#pragma unroll
+        for (int t = q; t < NTILE; ++t) z[t] = tile_mac<false, TF>(Y, n, 16 * t, n, 16 * q, nk, t1, z[t], li, lk, true);
+    }
+    if (c < n) {
+        TF* Q = I.fac + f.Qt + (int64_t)c * n;
+#pragma unroll
+        for (int t = 0; t < NTILE; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * t + MF::row(lk, r);
+                if (row < n) Q[row] = z[t][r];
+            }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2862,6 +3094,23 @@ hipError_t launch_ulv_qform(const FInst<T>* insts, const WorkItem* work, int nwo
     return hipGetLastError();
 }
 template <typename T>
+hipError_t launch_ulv_forms_w(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, int max_kx, int max_n,
+                              hipStream_t st) {
+    if (nwork <= 0) return hipSuccess;
+    if (max_m > FORM_W_ROWS || max_n > FORM_W_ROWS) return hipErrorInvalidValue;
+    const bool small = max_m <= 64;
+    const int gy = (max_kx + 63) / 64, qy = (max_n + 63) / 64;
+    if (gy > 0) {
+        if (small) klaunch((k_ulv_gform_w<T, 4>), dim3(nwork, gy), dim3(256), 0, st, insts, work);
+        else klaunch((k_ulv_gform_w<T, 8>), dim3(nwork, gy), dim3(256), 0, st, insts, work);
+    }
+    if (qy > 0) {
+        if (small) klaunch((k_ulv_qform_w<T, 4>), dim3(nwork, qy), dim3(256), 0, st, insts, work);
+        else klaunch((k_ulv_qform_w<T, 8>), dim3(nwork, qy), dim3(256), 0, st, insts, work);
+    }
+    return hipGetLastError();
+}
+template <typename T>
 hipError_t launch_ulv_rinv(const FInst<T>* insts, const WorkItem* work, int nwork, int max_cols, size_t lds,
                            hipStream_t st) {
     if (nwork <= 0 || max_cols <= 0) return hipSuccess;
@@ -3640,6 +3889,7 @@ template hipError_t launch_ulv_root<float>(const FInst<float>*, const WorkItem*,
 #define HSS_INST_SOLVE(T)                                                                                      \
     template hipError_t launch_ulv_gform<T>(const FInst<T>*, const WorkItem*, int, int, size_t, hipStream_t);       \
     template hipError_t launch_ulv_qform<T>(const FInst<T>*, const WorkItem*, int, int, size_t, hipStream_t);       \
+    template hipError_t launch_ulv_forms_w<T>(const FInst<T>*, const WorkItem*, int, int, int, int, hipStream_t);   \
     template hipError_t launch_ulv_gup<T>(const SInst<T>*, const SweepRec*, int, int, int, hipStream_t);            \
     template hipError_t launch_ulv_groot<T>(const SInst<T>*, const SweepRec*, int, int, size_t, int, hipStream_t);   \
     template hipError_t launch_ulv_rinv<T>(const FInst<T>*, const WorkItem*, int, int, size_t, hipStream_t);       \

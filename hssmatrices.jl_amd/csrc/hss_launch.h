@@ -48,6 +48,11 @@ hipError_t launch_ulv_wy(const FInst<T>* insts, const WorkItem* work, int nwork,
 template <typename T>
 hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwork, hipStream_t st);
 // solve operators, once per factorization (every non-root node in one launch)
+// Gz, Gr and Qt of nodes with at most FORM_W_ROWS rows (k_ulv_gform_w, k_ulv_qform_w)
+constexpr int FORM_W_ROWS = 128;
+template <typename T>
+hipError_t launch_ulv_forms_w(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, int max_kx, int max_n,
+                              hipStream_t st);
 template <typename T>
 hipError_t launch_ulv_gform(const FInst<T>* insts, const WorkItem* work, int nwork, int max_kx, size_t lds,
                             hipStream_t st);

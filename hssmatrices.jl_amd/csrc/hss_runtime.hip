@@ -1962,12 +1962,10 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
     FInst<TF>* d_inst = nullptr;
     WorkItem* d_work = nullptr;
     size_t lds_gform = 0, lds_qform = 0, lds_rinv = 0;
-    int max_kx = 0, max_nq = 0, max_rcols = 0;
+    int max_rcols = 0;
     for (auto* F : out) {
         lds_gform = std::max(lds_gform, F->lds_gform);
         lds_qform = std::max(lds_qform, F->lds_qform);
-        max_kx = std::max(max_kx, F->max_kx);
-        max_nq = std::max(max_nq, F->max_nq);
         const FNode& r = F->hfn[0];
         if (r.Dinv >= 0) {
             max_rcols = std::max(max_rcols, std::max(r.m, r.Kx));
@@ -2014,7 +2012,27 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
         return want && lev_n[h] <= 128 && lev_rows[h] <= factor_mf_max_rows((int)sizeof(TF)) &&
                lev_lds_mf[h] <= 160 * 1024;
     };
-    const int wy_count = (int)work.size();  // every non-root node of every matrix
+    const int nonroot = (int)work.size();  // every non-root node of every matrix
+    // The operator-forming kernels by size: a wave per 16 columns with the rows in registers
+    // up to 64 and up to FORM_W_ROWS rows (a 64-row node in the 128-row build would run twice
+    // the tiles), the LDS kernels beyond.
+    struct FormClass {
+        Range r;
+        int m = 0, kx = 0, nq = 0;
+    } form[3];
+    for (int c = 0; c < 3; ++c) {
+        form[c].r.off = (int)work.size();
+        for (int e = 0; e < nonroot; ++e) {
+            const WorkItem w = work[e];
+            const FNode& f = out[w.inst]->hfn[w.node];
+            if ((f.m <= 64 ? 0 : f.m <= FORM_W_ROWS ? 1 : 2) != c) continue;
+            work.push_back(w);
+            form[c].m = std::max(form[c].m, f.m);
+            form[c].kx = std::max(form[c].kx, f.Kx + f.nk);
+            if (f.Qt >= 0) form[c].nq = std::max(form[c].nq, f.n);
+        }
+        form[c].r.count = (int)work.size() - form[c].r.off;
+    }
     Range roots{(int)work.size(), cnt};
     for (int b = 0; b < cnt; ++b) work.push_back(WorkItem{b, 0});
     std::vector<FInst<TF>> hinst(cnt);
@@ -2050,9 +2068,10 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
                 HIP_TRY((launch_ulv_factor<TF>(d_inst, d_work + lev[h].off, lev[h].count, lev_lds[h], lev_thr[h], st)));
             }
         }
-        {
-            ProfScope ps("k_ulv_wy", 0, wy_count, st);
-            HIP_TRY((launch_ulv_wy<TF>(d_inst, d_work, wy_count, st)));
+        for (int h = 0; h < maxh; ++h) {
+            if (use_mf(h)) continue;  // that kernel writes these blocks itself
+            ProfScope ps("k_ulv_wy", h, lev[h].count, st);
+            HIP_TRY((launch_ulv_wy<TF>(d_inst, d_work + lev[h].off, lev[h].count, st)));
         }
         {
             ProfScope ps("k_ulv_root", 0, roots.count, st);
@@ -2063,13 +2082,15 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
             HIP_TRY((launch_ulv_rinv<TF>(d_inst, d_work + roots.off, roots.count, max_rcols, lds_rinv, st)));
         }
         // solve operators G and Qt of every non-root node (one launch each)
-        {
-            ProfScope ps("k_ulv_gform", 0, wy_count, st);
-            HIP_TRY((launch_ulv_gform<TF>(d_inst, d_work, wy_count, max_kx, lds_gform, st)));
+        for (int c = 0; c < 2; ++c) {
+            ProfScope ps("k_ulv_forms", c, form[c].r.count, st);
+            HIP_TRY((launch_ulv_forms_w<TF>(d_inst, d_work + form[c].r.off, form[c].r.count, form[c].m, form[c].kx,
+                                            form[c].nq, st)));
         }
-        {
-            ProfScope ps("k_ulv_qform", 0, wy_count, st);
-            HIP_TRY((launch_ulv_qform<TF>(d_inst, d_work, wy_count, max_nq, lds_qform, st)));
+        if (form[2].r.count > 0) {
+            ProfScope ps("k_ulv_gform", 0, form[2].r.count, st);
+            HIP_TRY((launch_ulv_gform<TF>(d_inst, d_work + form[2].r.off, form[2].r.count, form[2].kx, lds_gform, st)));
+            HIP_TRY((launch_ulv_qform<TF>(d_inst, d_work + form[2].r.off, form[2].r.count, form[2].nq, lds_qform, st)));
         }
         HIP_TRY(hipEventRecord(ctx->ev1, st));
         HIP_TRY(hipStreamSynchronize(st));
