@@ -161,7 +161,8 @@ struct FInst {
     const DevNode HSS_GLOBAL* nodes;
     const FNode HSS_GLOBAL* fn;
     const double HSS_GLOBAL* blob;
-    TF HSS_GLOBAL* fac;
+    TF HSS_GLOBAL* fac;  // resident: G, Qt and every root block
+    TF HSS_GLOBAL* tmp;  // the other factor blocks (Yql .. Vt, a non-root node's P12 and P21)
     TF HSS_GLOBAL* rw;
     int32_t HSS_GLOBAL* ipiv;
     int32_t HSS_GLOBAL* status;  // first zero pivot (1-based) of the root LU, 0 = none

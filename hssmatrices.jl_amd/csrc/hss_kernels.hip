@@ -435,12 +435,10 @@ __device__ __forceinline__ T merged_D(const ChildRed<T>& a, const ChildRed<T>& b
     return s;
 }
 
-// P12 = U1 B12 (mr1 x kv2), P21 = U2 B21 (mr2 x kv1) into global factor storage.
+// P12 = U1 B12 (mr1 x kv2), P21 = U2 B21 (mr2 x kv1) into global memory.
 template <typename T>
-__device__ void merge_products(const FInst<T>& I, const DevNode& nd, const FNode& f, const ChildRed<T>& a,
-                               const ChildRed<T>& b) {
-    T* P12 = I.fac + f.P12;
-    T* P21 = I.fac + f.P21;
+__device__ void merge_products(const FInst<T>& I, const DevNode& nd, const ChildRed<T>& a, const ChildRed<T>& b, T* P12,
+                               T* P21) {
     for (int e = threadIdx.x; e < a.mr * b.kv; e += blockDim.x) {
         const int r = e % a.mr, c = e / a.mr;
         T s = T(0);
@@ -529,7 +527,7 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
                 stage_to(sU, x.mr * x.ku, [&](int e) { return x.U[e]; });
                 stage_to(sB, x.ku * o.kv, [&](int e) { return gen<T>(I.blob, half ? nd.B21 : nd.B12, e); });
                 __syncthreads();
-                T* Pg = I.fac + (half ? f.P21 : f.P12);
+                T* Pg = I.tmp + (half ? f.P21 : f.P12);
                 for (int e = tid; e < nP; e += blockDim.x) {
                     const int rr = e % x.mr, c = e / x.mr;
                     T sum = T(0);
@@ -592,11 +590,11 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
             Wm = Wmw;
             __threadfence_block();
         } else {
-            merge_products(I, nd, f, a, b);
+            T* P12 = I.tmp + f.P12;
+            T* P21 = I.tmp + f.P21;
+            merge_products(I, nd, a, b, P12, P21);
             __threadfence_block();
             __syncthreads();
-            const T* P12 = I.fac + f.P12;
-            const T* P21 = I.fac + f.P21;
             for (int e = tid; e < R * n; e += blockDim.x) {
                 const int rr = e / n, c = e % n;
                 T val;
@@ -711,7 +709,7 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
         return i < p ? Us[i + (int64_t)j * m] : (i == p ? T(1) : T(0));
     };
     {
-        T* Y = I.fac + f.Yql;
+        T* Y = I.tmp + f.Yql;
         for (int e = tid; e < m * k; e += blockDim.x) Y[e] = yql(e % m, e / m);
         T* Ur = I.rw + f.rwU;  // reduced U = tril(U[m-k:m, :]), k x ku (ku == k here)
         for (int e = tid; e < k * ku; e += blockDim.x) {
@@ -748,7 +746,7 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
     }
     __syncthreads();
     {
-        T* Tg = I.fac + f.Tql;
+        T* Tg = I.tmp + f.Tql;
         for (int e = tid; e < k * k; e += blockDim.x) Tg[e] = Tq[e];
     }
 
@@ -914,8 +912,8 @@ __global__ __launch_bounds__(NT) void k_ulv_factor(const FInst<T>* __restrict__ 
     // ---- phase 5: outputs ----
     if (row_on) {
         if (r < nk) {
-            T* L1 = I.fac + f.L1;
-            T* Y = I.fac + f.Ylq;
+            T* L1 = I.tmp + f.L1;
+            T* Y = I.tmp + f.Ylq;
 #pragma unroll
             for (int q = 0; q < CPT; ++q) {
                 const int c = c0 + q;
@@ -925,7 +923,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor(const FInst<T>* __restrict__ 
                 }
             }
         } else if (r < m) {
-            T* L2a = I.fac + f.L2a;
+            T* L2a = I.tmp + f.L2a;
             T* Dr = I.rw + f.rwD;
             const int rr = r - nk;
 #pragma unroll
@@ -937,7 +935,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor(const FInst<T>* __restrict__ 
                 }
             }
         } else {
-            T* Vt = I.fac + f.Vt;
+            T* Vt = I.tmp + f.Vt;
             T* Vr = I.rw + f.rwV;
             const int j = r - m;
 #pragma unroll
@@ -951,7 +949,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor(const FInst<T>* __restrict__ 
         }
     }
     // LQ reflector scalars for the compact-WY blocks (built by k_ulv_wy)
-    for (int e = tid; e < nk; e += blockDim.x) I.fac[f.taulq + e] = taus[e];
+    for (int e = tid; e < nk; e += blockDim.x) I.tmp[f.taulq + e] = taus[e];
 }
 
 // LDS and sizes of the blocked LQ of k_ulv_factor_mf (its comment has the layouts).
@@ -1172,7 +1170,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
     constexpr int TPP = LqPanel<T>::TPP;
     T* Ts = Vs + 2 * 16 * NCP;
     T* tl = Ts + 2 * 16 * TPP;              // nk taus (nk <= n <= 128)
-    lq_panels<T, NTILE, 0>(a, LqPanel<T>{Vs, Ts, tl, I.fac + f.Tlq, nk, wave, lane});
+    lq_panels<T, NTILE, 0>(a, LqPanel<T>{Vs, Ts, tl, I.tmp + f.Tlq, nk, wave, lane});
     // Inverse of L1's diagonal block `wave`, which this wave holds: lane li solves L x = e_li.
     // (A kernel of its own after the factor, which also formed T again, took 245 us on 1022
     // nodes, one wave a block and its operands from memory.)
@@ -1191,7 +1189,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
             const T dii = lane_read(d[MF::reg_of(i)], 16 * MF::lane_of(i) + i);
             x[i] = i < nb && li < nb ? s / dii : T(0);
         }
-        T* Lig = I.fac + f.L1inv + (int64_t)wave * NB * NB;
+        T* Lig = I.tmp + f.L1inv + (int64_t)wave * NB * NB;
         if (lk == 0) {
 #pragma unroll
             for (int q = 0; q < 16; ++q) Lig[q + li * NB] = x[q];
@@ -1214,20 +1212,20 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
                 if (c >= n) continue;
                 const T x = a[t][r];
                 if (row < nk) {
-                    if (c < nk) I.fac[f.L1 + row + (int64_t)c * nk] = (c <= row) ? x : T(0);
-                    I.fac[f.Ylq + c + (int64_t)row * n] = (c < row) ? T(0) : (c == row ? T(1) : x);
+                    if (c < nk) I.tmp[f.L1 + row + (int64_t)c * nk] = (c <= row) ? x : T(0);
+                    I.tmp[f.Ylq + c + (int64_t)row * n] = (c < row) ? T(0) : (c == row ? T(1) : x);
                 } else if (row < m) {
                     const int rr = row - nk;
-                    if (c < nk) I.fac[f.L2a + rr + (int64_t)c * k] = x;
+                    if (c < nk) I.tmp[f.L2a + rr + (int64_t)c * k] = x;
                     else I.rw[f.rwD + rr + (int64_t)(c - nk) * f.mr] = x;
                 } else {
                     const int j = row - m;
-                    if (c < nk) I.fac[f.Vt + c + (int64_t)j * nk] = x;
+                    if (c < nk) I.tmp[f.Vt + c + (int64_t)j * nk] = x;
                     else I.rw[f.rwV + (c - nk) + (int64_t)j * f.nr] = x;
                 }
             }
     }
-    for (int e = tid; e < nk; e += blockDim.x) I.fac[f.taulq + e] = tl[e];
+    for (int e = tid; e < nk; e += blockDim.x) I.tmp[f.taulq + e] = tl[e];
 }
 
 // Compact-WY T blocks of the LQ reflectors (dlarft, forward columnwise) and the
@@ -1242,14 +1240,14 @@ __global__ __launch_bounds__(256) void k_ulv_wy(const FInst<T>* __restrict__ ins
     const int n = f.n, nk = f.nk;
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const int nwaves = blockDim.x / 64;
-    const T* taus = I.fac + f.taulq;
+    const T* taus = I.tmp + f.taulq;
     for (int bblk = wave; bblk < f.nblk; bblk += nwaves) {
         const int b0 = bblk * NB;
         const int nb = min(NB, nk - b0);
-        const T* Y = I.fac + f.Ylq;
-        const T* L1 = I.fac + f.L1;
-        T* Tb = I.fac + f.Tlq + (int64_t)bblk * NB * NB;
-        T* Li = I.fac + f.L1inv + (int64_t)bblk * NB * NB;
+        const T* Y = I.tmp + f.Ylq;
+        const T* L1 = I.tmp + f.L1;
+        T* Tb = I.tmp + f.Tlq + (int64_t)bblk * NB * NB;
+        T* Li = I.tmp + f.L1inv + (int64_t)bblk * NB * NB;
         // Gram of the block (strict upper part): G[a][b] = y_{b0+a} . y_{b0+b}
         T g[4];
 #pragma unroll
@@ -1334,11 +1332,11 @@ __global__ __launch_bounds__(1024) void k_ulv_root(const FInst<T>* __restrict__ 
     } else {
         const ChildRed<T> a = child_red(I, nd.left);
         const ChildRed<T> b = child_red(I, nd.right);
-        merge_products(I, nd, f, a, b);
+        T* P12 = I.fac + f.P12;
+        T* P21 = I.fac + f.P21;
+        merge_products(I, nd, a, b, P12, P21);
         __threadfence_block();
         __syncthreads();
-        const T* P12 = I.fac + f.P12;
-        const T* P21 = I.fac + f.P21;
         for (int e = tid; e < m * m; e += blockDim.x) A[e] = merged_D(a, b, P12, P21, e % m, e / m);
     }
     __threadfence_block();
@@ -1467,7 +1465,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_ulv_gform(const FInst<TF>* __
     for (int c = max(j0, Kx); c < min(j0 + RHS_TILE, Kx + nk); ++c) {
         const int l = c - Kx;
         for (int i = threadIdx.x; i < R; i += blockDim.x)
-            Gr[i + (int64_t)c * R] = i < mr ? -I.fac[f.L2a + i + (int64_t)l * f.k] : I.fac[f.Vt + l + (int64_t)(i - mr) * nk];
+            Gr[i + (int64_t)c * R] = i < mr ? -I.tmp[f.L2a + i + (int64_t)l * f.k] : I.tmp[f.Vt + l + (int64_t)(i - mr) * nk];
     }
     if (j0 >= Kx) return;
     const int nt = min(RHS_TILE, Kx - j0);
@@ -1501,9 +1499,9 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_ulv_gform(const FInst<TF>* __
     if (!nd.is_leaf) {
         // b = [b_1 - P12 u_2; b_2 - P21 u_1]   (ulvfactor.jl:74)
         const int mrr = m - mrl;
-        mfma_gemm<false, TF>(mrl, kvr, I.fac + f.P12, mrl, us + kvl * NTP, nt,
+        mfma_gemm<false, TF>(mrl, kvr, I.tmp + f.P12, mrl, us + kvl * NTP, nt,
                          [&](int i, int j, TF v) { bv[i * NTP + j] -= v; }, NTP);
-        mfma_gemm<false, TF>(mrr, kvl, I.fac + f.P21, mrr, us, nt,
+        mfma_gemm<false, TF>(mrr, kvl, I.tmp + f.P21, mrr, us, nt,
                          [&](int i, int j, TF v) { bv[(mrl + i) * NTP + j] -= v; }, NTP);
         __syncthreads();
     }
@@ -1511,20 +1509,20 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_ulv_gform(const FInst<TF>* __
     if (!f.pass) {
         // b <- Q_ql' b = b - Y (T (Y' b))   (ulvfactor.jl:42)
         if (k > 0) {
-            mfma_gemm<true, TF>(k, m, I.fac + f.Yql, m, bv, nt, [&](int i, int j, TF v) { t1[i * NTP + j] = v; }, NTP);
+            mfma_gemm<true, TF>(k, m, I.tmp + f.Yql, m, bv, nt, [&](int i, int j, TF v) { t1[i * NTP + j] = v; }, NTP);
             __syncthreads();
-            mfma_gemm<false, TF>(k, k, I.fac + f.Tql, k, t1, nt, [&](int i, int j, TF v) { t2[i * NTP + j] = v; }, NTP);
+            mfma_gemm<false, TF>(k, k, I.tmp + f.Tql, k, t1, nt, [&](int i, int j, TF v) { t2[i * NTP + j] = v; }, NTP);
             __syncthreads();
-            mfma_gemm<false, TF>(m, k, I.fac + f.Yql, m, t2, nt, [&](int i, int j, TF v) { bv[i * NTP + j] -= v; }, NTP);
+            mfma_gemm<false, TF>(m, k, I.tmp + f.Yql, m, t2, nt, [&](int i, int j, TF v) { bv[i * NTP + j] -= v; }, NTP);
             __syncthreads();
         }
         // zloc = L1 \ b[0:nk]  (ulvfactor.jl:48), blocked with inverted diagonal blocks
         for (int bb = 0; bb < f.nblk; ++bb) {
             const int b0 = bb * NB, nb = min(NB, nk - b0);
-            mfma_gemm<false, TF>(nb, b0, I.fac + f.L1 + b0, nk, zl, nt,
+            mfma_gemm<false, TF>(nb, b0, I.tmp + f.L1 + b0, nk, zl, nt,
                              [&](int i, int j, TF v) { t1[i * NTP + j] = bv[(b0 + i) * NTP + j] - v; }, NTP);
             __syncthreads();
-            mfma_gemm<false, TF>(nb, nb, I.fac + f.L1inv + (int64_t)bb * NB * NB, NB, t1, nt,
+            mfma_gemm<false, TF>(nb, nb, I.tmp + f.L1inv + (int64_t)bb * NB * NB, NB, t1, nt,
                              [&](int i, int j, TF v) { zl[(b0 + i) * NTP + j] = v; }, NTP);
             __syncthreads();
         }
@@ -1574,10 +1572,10 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_ulv_qform(const FInst<TF>* __
     __syncthreads();
     for (int bb = f.nblk - 1; bb >= 0; --bb) {
         const int b0 = bb * NB, nb = min(NB, nk - b0);
-        const TF* Yb = I.fac + f.Ylq + (int64_t)b0 * n + b0;  // rows b0.., columns b0..b0+nb
+        const TF* Yb = I.tmp + f.Ylq + (int64_t)b0 * n + b0;  // rows b0.., columns b0..b0+nb
         mfma_gemm<true, TF>(nb, n - b0, Yb, n, z + b0 * NTP, nt, [&](int i, int j, TF v) { t1[i * NTP + j] = v; }, NTP);
         __syncthreads();
-        mfma_gemm<false, TF>(nb, nb, I.fac + f.Tlq + (int64_t)bb * NB * NB, NB, t1, nt,
+        mfma_gemm<false, TF>(nb, nb, I.tmp + f.Tlq + (int64_t)bb * NB * NB, NB, t1, nt,
                          [&](int i, int j, TF v) { t2[i * NTP + j] = v; }, NTP);
         __syncthreads();
         mfma_gemm<false, TF>(n - b0, nb, Yb, n, t2, nt, [&](int i, int j, TF v) { z[(b0 + i) * NTP + j] -= v; }, NTP);
@@ -1632,7 +1630,7 @@ __global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_gform_w(const F
     for (int c = max(j0, Kx); c < min(j0 + 16, Kx + nk); ++c) {
         const int l = c - Kx;
         for (int i = lane; i < R; i += 64)
-            Gr[i + (int64_t)c * R] = i < mr ? -I.fac[f.L2a + i + (int64_t)l * k] : I.fac[f.Vt + l + (int64_t)(i - mr) * nk];
+            Gr[i + (int64_t)c * R] = i < mr ? -I.tmp[f.L2a + i + (int64_t)l * k] : I.tmp[f.Vt + l + (int64_t)(i - mr) * nk];
     }
     if (j0 >= Kx) return;
     const int c = j0 + li;  // this lane's input column
@@ -1640,21 +1638,21 @@ __global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_gform_w(const F
     // b for x = e_c: a unit row, or (u_1, u_2) a column of -P21 or -P12 over rows [p0, p1);
     // (ulvfactor.jl:74: b = [b_1 - P12 u_2; b_2 - P21 u_1])
     int unit = on && nd.is_leaf ? c : -1, p0 = 0, p1 = 0, wl = 0;
-    const TF* pc = I.fac;
+    const TF* pc = I.tmp;
     const double* wc = nullptr;  // W' e_l is row l of W (wl rows)
     if (on && !nd.is_leaf) {
         const DevNode dl = I.nodes[nd.left], dr = I.nodes[nd.right];
         const int mrl = I.fn[nd.left].mr;
         if (c < mrl) unit = c;
         else if (c < mrl + dl.kv) {
-            pc = I.fac + f.P21 + (int64_t)(c - mrl) * (m - mrl);
+            pc = I.tmp + f.P21 + (int64_t)(c - mrl) * (m - mrl);
             p0 = mrl;
             p1 = m;
             wc = I.blob + dl.W + (c - mrl);
             wl = dl.kv;
         } else if (c < m + dl.kv) unit = c - dl.kv;
         else {
-            pc = I.fac + f.P12 + (int64_t)(c - m - dl.kv) * mrl;
+            pc = I.tmp + f.P12 + (int64_t)(c - m - dl.kv) * mrl;
             p1 = mrl;
             wc = I.blob + dr.W + (c - m - dl.kv);
             wl = dr.kv;
@@ -1672,8 +1670,8 @@ __global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_gform_w(const F
         }
     if (!f.pass && k > 0) {
         // b <- Q_ql' b = b - Y (T (Y' b))   (ulvfactor.jl:42)
-        const TF* Y = I.fac + f.Yql;
-        const TF* Tq = I.fac + f.Tql;
+        const TF* Y = I.tmp + f.Yql;
+        const TF* Tq = I.tmp + f.Tql;
         V4 t1[NTILE];
 #pragma unroll
         for (int q = 0; q < NTILE; ++q) {
@@ -1722,14 +1720,14 @@ __global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_gform_w(const F
     }
     // zloc = L1 \ b[0:nk]  (ulvfactor.jl:48), blocked with inverted diagonal blocks (whose
     // columns beyond nk are zero); zloc replaces b tile by tile
-    const TF* L1 = I.fac + f.L1;
+    const TF* L1 = I.tmp + f.L1;
 #pragma unroll
     for (int q = 0; q < NTILE; ++q) {
         if (16 * q >= nk) continue;
         V4 s = b[q];
 #pragma unroll
         for (int t = 0; t < q; ++t) s = tile_mac<false, TF>(L1, nk, 16 * q, nk, 16 * t, nk, b[t], s, li, lk, true);
-        b[q] = tile_mac<false, TF>(I.fac + f.L1inv + (int64_t)q * NB * NB, NB, 0, NB, 0, NB, s, V4{TF(0), TF(0), TF(0), TF(0)},
+        b[q] = tile_mac<false, TF>(I.tmp + f.L1inv + (int64_t)q * NB * NB, NB, 0, NB, 0, NB, s, V4{TF(0), TF(0), TF(0), TF(0)},
                                    li, lk, false);
     }
     if (on) {
@@ -1765,14 +1763,14 @@ __global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_qform_w(const F
     for (int t = 0; t < NTILE; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) z[t][r] = 16 * t + MF::row(lk, r) == c ? TF(1) : TF(0);
-    const TF* Y = I.fac + f.Ylq;
+    const TF* Y = I.tmp + f.Ylq;
 #pragma unroll
     for (int q = NTILE - 1; q >= 0; --q) {
         if (16 * q >= nk || 16 * q > j0) continue;
         V4 t1 = {TF(0), TF(0), TF(0), TF(0)};
 #pragma unroll
         for (int t = q; t < NTILE; ++t) t1 = tile_mac<true, TF>(Y, n, 16 * q, nk, 16 * t, n, z[t], t1, li, lk, false);
-        t1 = tile_mac<false, TF>(I.fac + f.Tlq + (int64_t)q * NB * NB, NB, 0, NB, 0, NB, t1, V4{TF(0), TF(0), TF(0), TF(0)}, li,
+        t1 = tile_mac<false, TF>(I.tmp + f.Tlq + (int64_t)q * NB * NB, NB, 0, NB, 0, NB, t1, V4{TF(0), TF(0), TF(0), TF(0)}, li,
                                  lk, false);
 #pragma unroll
         for (int t = q; t < NTILE; ++t) z[t] = tile_mac<false, TF>(Y, n, 16 * t, n, 16 * q, nk, t1, z[t], li, lk, true);

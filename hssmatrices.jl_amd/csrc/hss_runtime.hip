@@ -157,7 +157,9 @@ struct SlotCache {
     char* d = nullptr;
     std::vector<char> h;
     int used = 0, next = 0;
-    ~SlotCache() { (void)hipFree(d); }
+    ~SlotCache() {
+        if (d) (void)hipFree(d);
+    }
     hipError_t get(const void* v, size_t bytes, hipStream_t st, const void** out) {
         if (!d) {
             rec = bytes;
@@ -273,6 +275,73 @@ static hss_status plan_create_impl(int32_t count, hss_fact_s* const* facts, cons
                                    const double* const* dB, const int64_t* ldb, double* const* dX, const int64_t* ldx,
                                    int32_t with_refinement, bool hold, hss_plan_t* out);
 
+// Device memory of factors and plans, which come and go with every `\`: blocks given back are
+// kept for the next request of about their size (at most twice it; sizes are rounded up to an
+// eighth of their power of two, so that matrices with slightly other ranks share them), up to
+// kHeldMax bytes and kHeldBlocks blocks in all, and freed with the context or when an allocation fails.  A block
+// is given back only once the context's stream is idle, as hipFree would have waited.  hipMalloc
+// and hipFree cost tens to hundreds of microseconds each (mapping and unmapping).
+class DevPool {
+public:
+    template <typename T>
+    hipError_t get(T** p, size_t bytes) {
+        *p = nullptr;
+        size_t step = 4096;
+        while (16 * step <= bytes) step *= 2;
+        bytes = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = held.lower_bound(bytes);
+        if (it != held.end() && it->first <= 2 * bytes) {
+            *p = static_cast<T*>(it->second);
+            held_bytes -= it->first;
+            used[it->second] = it->first;
+            held.erase(it);
+            return hipSuccess;
+        }
+        void* d = nullptr;
+        hipError_t e = hipMalloc(&d, bytes);
+        if (e != hipSuccess && !held.empty()) {
+            (void)hipGetLastError();
+            trim_locked();
+            e = hipMalloc(&d, bytes);
+        }
+        if (e != hipSuccess) return e;
+        used[d] = bytes;
+        *p = static_cast<T*>(d);
+        return hipSuccess;
+    }
+    void put(void* p, hipStream_t st) {
+        if (!p) return;
+        (void)hipStreamSynchronize(st);
+        std::lock_guard<std::mutex> lk(mu);
+        const auto it = used.find(p);
+        const size_t bytes = it->second;
+        used.erase(it);
+        if (held_bytes + bytes > kHeldMax || held.size() >= kHeldBlocks) {
+            (void)hipFree(p);
+            return;
+        }
+        held.emplace(bytes, p);
+        held_bytes += bytes;
+    }
+    void trim() {
+        std::lock_guard<std::mutex> lk(mu);
+        trim_locked();
+    }
+
+private:
+    static constexpr size_t kHeldMax = size_t(2) << 30, kHeldBlocks = 512;
+    void trim_locked() {
+        for (auto& h : held) (void)hipFree(h.second);
+        held.clear();
+        held_bytes = 0;
+    }
+    std::mutex mu;
+    std::multimap<size_t, void*> held;
+    std::map<void*, size_t> used;
+    size_t held_bytes = 0;
+};
+
 // Handles hold references on what they use (a matrix on its context, a factor on
 // its matrix, a plan on its factors and context, a server on its context), so
 // destroying them in any order -- as garbage-collected bindings do -- is safe: a
@@ -282,6 +351,7 @@ struct hss_ctx_s {
     int device = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    DevPool pool;
 };
 
 struct hss_mat_s {
@@ -325,11 +395,11 @@ struct hss_fact_s {
     hss_mat_s* mat = nullptr;
     hss_prec prec = HSS_PREC_FP64;
     std::vector<FNode> hfn;
+    // one allocation, at d_fac: the resident operators, d_fn, d_swork, d_piv
     FNode* d_fn = nullptr;
     void* d_fac = nullptr;
-    int64_t fac_len = 0;
+    int64_t tmp_len = 0;               // factorization-time data, released with the factorization
     int32_t* d_piv = nullptr;
-    int32_t* d_status = nullptr;
     int64_t res_len = 0;               // resident part of the factor (G, Qt, root LU)
     int64_t yrows = 0, zrows = 0;      // solve workspace rows (times nrhs)
     size_t lds_groot = 0;              // LDS of the root solve kernel
@@ -337,7 +407,6 @@ struct hss_fact_s {
     size_t lds_groot2 = 0;             // the inverse-and-refine root kernel (0: not available)
     size_t lds_groot2s = 0;            // the same with D and Mb staged too
     size_t lds_gform = 0, lds_qform = 0;
-    int max_kx = 0, max_nq = 0;        // widest Gr / Qt (columns formed per node)
     void* d_wy = nullptr;  // y blocks, then the z blocks at wy + yrows * nrhs
     size_t ws_cap = 0;     // nrhs capacity
     SlotCache sinst;
@@ -409,6 +478,7 @@ static void ctx_release(hss_ctx_s* c) {
     if (!c || --c->refs > 0) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    c->pool.trim();
     (void)hipEventDestroy(c->ev0);
     (void)hipEventDestroy(c->ev1);
     (void)hipStreamDestroy(c->stream);
@@ -473,8 +543,10 @@ static void free_mat(hss_mat_s* M) {
     (void)hipFree(M->d_nodes);
     (void)hipFree(M->d_work);
     (void)hipFree(M->d_Z);
-    (void)hipFree(M->d_io_b);
-    (void)hipFree(M->d_io_c);
+    if (M->ctx) {
+        M->ctx->pool.put(M->d_io_b, M->ctx->stream);
+        M->ctx->pool.put(M->d_io_c, M->ctx->stream);
+    }
     (void)hipFree(M->d_cutT);
     (void)hipFree(M->d_cut);
     delete M;
@@ -1663,14 +1735,14 @@ extern "C" hss_status hss_matmul_dev(hss_mat_t M, int32_t nrhs, double alpha, co
     return matmul_enqueue(M, nrhs, alpha, dB, ldb, beta, dC, ldc);
 }
 
-static hss_status ensure_io(double** a, double** b, size_t* cap, size_t need) {
+static hss_status ensure_io(hss_ctx_s* ctx, double** a, double** b, size_t* cap, size_t need) {
     if (need <= *cap) return HSS_OK;
-    (void)hipFree(*a);
-    (void)hipFree(*b);
+    ctx->pool.put(*a, ctx->stream);
+    ctx->pool.put(*b, ctx->stream);
     *a = *b = nullptr;
     *cap = 0;
-    HIP_TRY(dalloc(a, need));
-    HIP_TRY(dalloc(b, need));
+    HIP_TRY(ctx->pool.get(a, need * sizeof(double)));
+    HIP_TRY(ctx->pool.get(b, need * sizeof(double)));
     *cap = need;
     return HSS_OK;
 }
@@ -1684,7 +1756,7 @@ extern "C" hss_status hss_matmul(hss_mat_t M, int32_t nrhs, double alpha, const 
         return fail(HSS_ERR_DIM, "leading dimension smaller than the matrix size");
     HIP_TRY(hipSetDevice(M->ctx->device));
     const int64_t nb = std::max<int64_t>(M->cols, 1), nc = std::max<int64_t>(M->rows, 1);
-    hss_status s = ensure_io(&M->d_io_b, &M->d_io_c, &M->io_cap, (size_t)std::max(nb, nc) * nrhs);
+    hss_status s = ensure_io(M->ctx, &M->d_io_b, &M->d_io_c, &M->io_cap, (size_t)std::max(nb, nc) * nrhs);
     if (s != HSS_OK) return s;
     hipStream_t st = M->ctx->stream;
     HIP_TRY(hipMemcpy2DAsync(M->d_io_b, nb * sizeof(double), B, ldb * sizeof(double), M->cols * sizeof(double), nrhs,
@@ -1723,8 +1795,8 @@ static size_t factor_lds(const FNode& f, const DevNode& d) {
 
 // Fill the factor metadata of one matrix; offsets are relative to this
 // matrix's own factor / workspace buffers.  The factor buffer holds the resident
-// solve operators first ([0, res_len): every G and Qt, the root's LU data and
-// couplings) and the factorization-time data after them.
+// solve operators ([0, res_len): every G and Qt, the root's LU data and couplings);
+// the factorization-time data is in a buffer of its own ([0, tmp_len)).
 template <typename TF>
 static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
     const int nn = M->nn;
@@ -1821,6 +1893,7 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
     }
     F->res_len = fac;
     // factorization-time data
+    fac = 0;
     int64_t rw = 0, yrows = 0, zrows = 0;
     for (int i = nn - 1; i >= 1; --i) {
         const DevNode& d = M->hn[i];
@@ -1845,7 +1918,7 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
         f.rwU = take(rw, (int64_t)f.mr * d.ku);
         f.rwV = take(rw, (int64_t)f.nr * d.kv);
     }
-    F->fac_len = fac;
+    F->tmp_len = fac;
     // solve workspace: y blocks of non-root nodes, z blocks of branches and the root
     for (int i = 0; i < nn; ++i) {
         FNode& f = F->hfn[i];
@@ -1856,7 +1929,6 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
     F->zrows = zrows;
     // LDS (rows of NTP = RHS_TILE columns) and widths of the operator-forming kernels
     size_t gform = 0, qform = 0, groot = 0;
-    int max_kx = 0, max_nq = 0;
     for (int i = 0; i < nn; ++i) {
         const FNode& f = F->hfn[i];
         const DevNode& d = M->hn[i];
@@ -1867,8 +1939,6 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
             const size_t tr = (size_t)std::max(std::max(f.k, NB), d.kv);
             gform = std::max(gform, (size_t)f.m + std::max(f.nk, 1) + kvc + 2 * tr);
             qform = std::max(qform, (size_t)f.n + 2 * NB);
-            max_kx = std::max(max_kx, f.Kx + f.nk);
-            if (f.Qt >= 0) max_nq = std::max(max_nq, f.n);
         }
     }
     const size_t tv = sizeof(TF) * RHS_TILE;
@@ -1881,8 +1951,6 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
         F->lds_groot2 = sizeof(TF) * (size_t)(((int64_t)fr.m * fr.m + 15) / 16 * 16 + io);
         F->lds_groot2s = sizeof(TF) * (size_t)((2 * (int64_t)fr.m * fr.m + (int64_t)fr.m * fr.Kx + 15) / 16 * 16 + io);
     }
-    F->max_kx = max_kx;
-    F->max_nq = max_nq;
     if (F->lds_gform > 160 * 1024 || F->lds_groot > 160 * 1024)
         return fail(HSS_ERR_UNSUPPORTED, "a node exceeds the LDS of the solve-operator kernels");
     return HSS_OK;
@@ -1891,22 +1959,39 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
 static void free_fact(hss_fact_s* F) {
     if (!F) return;
     destroy_plan_cache(F->plan_cache);
-    (void)hipFree(F->d_fn);
-    (void)hipFree(F->d_fac);
-    (void)hipFree(F->d_piv);
-    (void)hipFree(F->d_status);
-    (void)hipFree(F->d_wy);
-    (void)hipFree(F->d_swork);
-    (void)hipFree(F->d_r);
-    (void)hipFree(F->d_d);
-    (void)hipFree(F->d_nrm);
-    (void)hipFree(F->d_gm);
-    (void)hipFree(F->d_io_b);
-    (void)hipFree(F->d_io_x);
+    hss_ctx_s* ctx = F->mat->ctx;
+    for (void* p : {F->d_fac, (void*)F->d_io_b, (void*)F->d_io_x}) ctx->pool.put(p, ctx->stream);
+    for (void* p : {F->d_wy, (void*)F->d_r, (void*)F->d_d, (void*)F->d_nrm, (void*)F->d_gm})
+        if (p) (void)hipFree(p);
     delete F;
 }
 
-static hss_status ensure_schedule(hss_fact_s* F);
+static void build_schedule(const std::vector<hss_fact_s*>& facts, Schedule& S);
+static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
+
+// The factor's own device memory, one allocation: the resident operators (16 elements of
+// slack for whole-vector loads), the node table, the single-request solve schedule (so that
+// solves, the allocation-free one included, find it ready) and the root's pivots.
+template <typename TF>
+static hss_status alloc_resident(hss_fact_s* F) {
+    build_schedule(std::vector<hss_fact_s*>{F}, F->sched);
+    const size_t fn_b = sizeof(FNode) * F->hfn.size(), sw_b = sizeof(SweepRec) * F->sched.rec.size();
+    const size_t at_fn = align256(sizeof(TF) * ((size_t)F->res_len + 16)), at_sw = align256(at_fn + fn_b),
+                 at_piv = align256(at_sw + sw_b), total = at_piv + sizeof(int32_t) * ((size_t)F->hfn[0].m + 1);
+    char* d = nullptr;
+    const hipError_t e = F->mat->ctx->pool.get(&d, total);
+    if (e != hipSuccess) return fail(HSS_ERR_OOM, std::string("factor allocation: ") + hipGetErrorString(e));
+    F->d_fac = d;
+    F->d_fn = reinterpret_cast<FNode*>(d + at_fn);
+    F->d_swork = reinterpret_cast<SweepRec*>(d + at_sw);
+    F->d_piv = reinterpret_cast<int32_t*>(d + at_piv);
+    std::vector<char> tab(at_sw - at_fn + sw_b);
+    std::memcpy(tab.data(), F->hfn.data(), fn_b);
+    std::memcpy(tab.data() + (at_sw - at_fn), F->sched.rec.data(), sw_b);
+    HIP_TRY(hipMemcpy(d + at_fn, tab.data(), tab.size(), hipMemcpyHostToDevice));
+    F->dev_bytes = (int64_t)(sizeof(TF) * F->res_len + fn_b + 4 * (F->hfn[0].m + 1));
+    return HSS_OK;
+}
 
 // Factor a batch of matrices that share one context: one launch per height
 // across all of them, then one root launch.
@@ -1916,8 +2001,8 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
     hss_ctx_s* ctx = mats[0]->ctx;
     hipStream_t st = ctx->stream;
     out.assign(cnt, nullptr);
-    std::vector<int64_t> rw_off(cnt), rw_len(cnt);
-    int64_t rw_total = 0;
+    std::vector<int64_t> rw_off(cnt), tmp_off(cnt);
+    int64_t rw_total = 0, tmp_total = 0;
     int maxh = 0;
     auto cleanup = [&]() {
         for (auto* f : out) free_fact(f);
@@ -1944,23 +2029,13 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
             rw = std::max(rw, f.rwU + (int64_t)f.mr * M->hn[i].ku);
         }
         rw_off[b] = rw_total;
-        rw_len[b] = rw;
-        rw_total += rw;
+        rw_total += (rw + 15) & ~int64_t(15);
         maxh = std::max(maxh, M->max_height);
-        hipError_t e;
-        if ((e = dalloc(&F->d_fn, F->hfn.size())) != hipSuccess ||
-            (e = dalloc(reinterpret_cast<TF**>(&F->d_fac), (size_t)F->fac_len)) != hipSuccess ||
-            (e = dalloc(&F->d_piv, (size_t)F->hfn[0].m)) != hipSuccess || (e = dalloc(&F->d_status, 1)) != hipSuccess) {
-            cleanup();
-            return fail(HSS_ERR_OOM, std::string("factor allocation: ") + hipGetErrorString(e));
-        }
-        HIP_TRY(hipMemcpyAsync(F->d_fn, F->hfn.data(), sizeof(FNode) * F->hfn.size(), hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemsetAsync(F->d_status, 0, sizeof(int32_t), st));
-        F->dev_bytes = (int64_t)(sizeof(TF) * F->fac_len + sizeof(FNode) * F->hfn.size() + 4 * (F->hfn[0].m + 1));
+        tmp_off[b] = tmp_total;
+        tmp_total += (F->tmp_len + 15) & ~int64_t(15);
+        s = alloc_resident<TF>(F);
+        if (s != HSS_OK) { cleanup(); return s; }
     }
-    TF* d_rw = nullptr;
-    FInst<TF>* d_inst = nullptr;
-    WorkItem* d_work = nullptr;
     size_t lds_gform = 0, lds_qform = 0, lds_rinv = 0;
     int max_rcols = 0;
     for (auto* F : out) {
@@ -2036,27 +2111,43 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
     Range roots{(int)work.size(), cnt};
     for (int b = 0; b < cnt; ++b) work.push_back(WorkItem{b, 0});
     std::vector<FInst<TF>> hinst(cnt);
-    hipError_t e;
-    if ((e = dalloc(&d_rw, (size_t)rw_total)) != hipSuccess || (e = dalloc(&d_inst, (size_t)cnt)) != hipSuccess ||
-        (e = dalloc(&d_work, work.size())) != hipSuccess) {
-        (void)hipFree(d_rw); (void)hipFree(d_inst); (void)hipFree(d_work);
+    // One allocation for everything that ends with this call: the instances and work items
+    // (one copy to the device), the status words (one copy back), rw and tmp.  Each hipMalloc,
+    // hipFree and small copy costs tens of microseconds, and hipFree waits for the device:
+    // with six allocations, four copies and a resized copy of the factor per matrix, factoring,
+    // solving and releasing 32 matrices took 26-35 ms, 5 ms of it kernels; now 4.2 ms.
+    const size_t inst_bytes = align256(sizeof(FInst<TF>) * cnt), work_bytes = align256(sizeof(WorkItem) * work.size());
+    const size_t info_bytes = align256(sizeof(int32_t) * cnt);
+    char* d_scratch = nullptr;
+    hipError_t e = ctx->pool.get(&d_scratch,
+                                 inst_bytes + work_bytes + info_bytes + sizeof(TF) * (size_t)(rw_total + tmp_total + 16));
+    if (e != hipSuccess) {
         cleanup();
         return fail(HSS_ERR_OOM, std::string("factor workspace: ") + hipGetErrorString(e));
     }
+    auto* d_inst = reinterpret_cast<FInst<TF>*>(d_scratch);
+    auto* d_work = reinterpret_cast<WorkItem*>(d_scratch + inst_bytes);
+    auto* d_info = reinterpret_cast<int32_t*>(d_scratch + inst_bytes + work_bytes);
+    auto* d_rw = reinterpret_cast<TF*>(d_scratch + inst_bytes + work_bytes + info_bytes);
+    TF* d_tmp = d_rw + rw_total;
     for (int b = 0; b < cnt; ++b) {
         FInst<TF>& I = hinst[b];
         I.nodes = mats[b]->d_nodes;
         I.fn = out[b]->d_fn;
         I.blob = mats[b]->d_blob;
         I.fac = reinterpret_cast<TF*>(out[b]->d_fac);
+        I.tmp = d_tmp + tmp_off[b];
         I.rw = d_rw + rw_off[b];
         I.ipiv = out[b]->d_piv;
-        I.status = out[b]->d_status;
+        I.status = d_info + b;
     }
+    std::vector<int32_t> info(cnt, 0);
     hss_status rs = HSS_OK;
     auto run = [&]() -> hss_status {
-        HIP_TRY(hipMemcpyAsync(d_inst, hinst.data(), sizeof(FInst<TF>) * cnt, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_work, work.data(), sizeof(WorkItem) * work.size(), hipMemcpyHostToDevice, st));
+        std::vector<char> tab(inst_bytes + sizeof(WorkItem) * work.size());
+        std::memcpy(tab.data(), hinst.data(), sizeof(FInst<TF>) * cnt);
+        std::memcpy(tab.data() + inst_bytes, work.data(), sizeof(WorkItem) * work.size());
+        HIP_TRY(hipMemcpyAsync(d_scratch, tab.data(), tab.size(), hipMemcpyHostToDevice, st));
         HIP_TRY(hipEventRecord(ctx->ev0, st));
         for (int h = 0; h < maxh; ++h) {
             if (use_mf(h)) {
@@ -2093,46 +2184,21 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
             HIP_TRY((launch_ulv_qform<TF>(d_inst, d_work + form[2].r.off, form[2].r.count, form[2].nq, lds_qform, st)));
         }
         HIP_TRY(hipEventRecord(ctx->ev1, st));
+        HIP_TRY(hipMemcpyAsync(info.data(), d_info, sizeof(int32_t) * cnt, hipMemcpyDeviceToHost, st));
         HIP_TRY(hipStreamSynchronize(st));
         float ms = 0.f;
         if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess) g_last_ms = ms;
         return HSS_OK;
     };
     rs = run();
-    (void)hipFree(d_rw);
-    (void)hipFree(d_inst);
-    (void)hipFree(d_work);
+    ctx->pool.put(d_scratch, st);
     if (rs != HSS_OK) { cleanup(); return rs; }
-    for (int b = 0; b < cnt; ++b) {
-        int32_t info = 0;
-        HIP_TRY(hipMemcpy(&info, out[b]->d_status, sizeof(int32_t), hipMemcpyDeviceToHost));
-        if (info != 0) {
+    for (int b = 0; b < cnt; ++b)
+        if (info[b] != 0) {
             cleanup();
-            return fail(HSS_ERR_SINGULAR, "SingularException(" + std::to_string(info) +
+            return fail(HSS_ERR_SINGULAR, "SingularException(" + std::to_string(info[b]) +
                                               "): exactly zero pivot in the root block of matrix " + std::to_string(b));
         }
-    }
-    // keep only the resident solve operators (the stream is idle here)
-    for (int b = 0; b < cnt; ++b) {
-        hss_fact_s* F = out[b];
-        TF* res = nullptr;
-        hipError_t e2 = dalloc(&res, (size_t)F->res_len + 16);
-        if (e2 != hipSuccess) {
-            cleanup();
-            return fail(HSS_ERR_OOM, std::string("factor allocation: ") + hipGetErrorString(e2));
-        }
-        HIP_TRY(hipMemcpy(res, F->d_fac, sizeof(TF) * (size_t)F->res_len, hipMemcpyDeviceToDevice));
-        (void)hipFree(F->d_fac);
-        F->d_fac = res;
-        F->fac_len = F->res_len;
-        F->dev_bytes = (int64_t)(sizeof(TF) * F->fac_len + sizeof(FNode) * F->hfn.size() + 4 * (F->hfn[0].m + 1));
-    }
-    // the single-request solve schedule, built here so that solves (the allocation-free one
-    // included) find it ready
-    for (int b = 0; b < cnt; ++b) {
-        hss_status s2 = ensure_schedule(out[b]);
-        if (s2 != HSS_OK) { cleanup(); return s2; }
-    }
     for (auto* F : out) F->mat->refs++;
     return HSS_OK;
 }
@@ -2423,21 +2489,10 @@ static hss_status launch_schedule(const SInst<TF>* di, const SweepRec* dw, const
     return HSS_OK;
 }
 
-static hss_status ensure_schedule(hss_fact_s* F) {
-    if (F->d_swork) return HSS_OK;
-    build_schedule(std::vector<hss_fact_s*>{F}, F->sched);
-    HIP_TRY(dalloc(&F->d_swork, F->sched.rec.size()));
-    HIP_TRY(hipMemcpy(F->d_swork, F->sched.rec.data(), sizeof(SweepRec) * F->sched.rec.size(),
-                      hipMemcpyHostToDevice));
-    return HSS_OK;
-}
-
 template <typename TF>
 static hss_status solve_one(hss_fact_s* F, int nrhs, const double* dB, int64_t ldb, double* dX, int64_t ldx,
                             hipStream_t st) {
     hss_status s = ensure_solve_ws<TF>(F, nrhs);
-    if (s != HSS_OK) return s;
-    s = ensure_schedule(F);
     if (s != HSS_OK) return s;
     SInst<TF> I = make_sinst<TF>(SolveReq{F, nrhs, dB, ldb, dX, ldx});
     const void* dv = nullptr;
@@ -2751,7 +2806,7 @@ extern "C" hss_status hss_ulv_solve(hss_fact_t F, int32_t nrhs, const double* B,
     if (ldb < M->rows || ldx < M->rows) return fail(HSS_ERR_DIM, "leading dimension smaller than the matrix size");
     HIP_TRY(hipSetDevice(M->ctx->device));
     const int64_t n = std::max<int64_t>(M->rows, 1);
-    hss_status s = ensure_io(&F->d_io_b, &F->d_io_x, &F->io_cap, (size_t)n * nrhs);
+    hss_status s = ensure_io(M->ctx, &F->d_io_b, &F->d_io_x, &F->io_cap, (size_t)n * nrhs);
     if (s != HSS_OK) return s;
     hipStream_t st = M->ctx->stream;
     HIP_TRY(hipMemcpy2DAsync(F->d_io_b, n * sizeof(double), B, ldb * sizeof(double), M->rows * sizeof(double), nrhs,
@@ -2843,22 +2898,14 @@ static void free_plan(hss_plan_s* P) {
     drop_ir_graphs(P);
     if (P->gexec) (void)hipGraphExecDestroy(P->gexec);
     if (P->graph) (void)hipGraphDestroy(P->graph);
-    (void)hipFree(P->arena);
-    (void)hipFree(P->d_sinst[0]);
-    (void)hipFree(P->d_sinst[1]);
-    (void)hipFree(P->d_mv);
-    (void)hipFree(P->d_vec);
-    (void)hipFree(P->d_work);
-    (void)hipFree(P->d_rec);
-    (void)hipFree(P->d_norms);
-    (void)hipFree(P->d_rel);
-    (void)hipFree(P->d_count);
+    for (void* p : {(void*)P->arena, (void*)P->d_sinst[0], (void*)P->d_sinst[1], (void*)P->d_rec})
+        P->ctx->pool.put(p, P->ctx->stream);
+    for (void* p : {(void*)P->d_mv, (void*)P->d_vec, (void*)P->d_work, (void*)P->d_norms, (void*)P->d_rel, (void*)P->d_count})
+        if (p) (void)hipFree(p);
     if (P->h_count) (void)hipHostFree(P->h_count);
     for (hipEvent_t e : P->count_ev) (void)hipEventDestroy(e);
     delete P;
 }
-
-static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 template <typename TF>
 static hss_status plan_tables(hss_plan_s* P) {
@@ -2882,7 +2929,7 @@ static hss_status plan_tables(hss_plan_s* P) {
             tot = align256(tot + sizeof(double) * (size_t)M->rows * q.nrhs);
         }
     }
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&P->arena), std::max<size_t>(tot, 256)));
+    HIP_TRY(P->ctx->pool.get(&P->arena, std::max<size_t>(tot, 256)));
     P->dev_bytes = (int64_t)tot;
     P->sinst_size = sizeof(SInst<TF>);
     for (int t = 0; t < (P->has_ir ? 2 : 1); ++t) {
@@ -2901,7 +2948,7 @@ static hss_status plan_tables(hss_plan_s* P) {
             v[i] = make_sinst<TF>(qq, ws);
         }
         P->h_sinst[t].assign(reinterpret_cast<char*>(v.data()), reinterpret_cast<char*>(v.data() + cnt));
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&P->d_sinst[t]), P->h_sinst[t].size()));
+        HIP_TRY(P->ctx->pool.get(&P->d_sinst[t], P->h_sinst[t].size()));
         HIP_TRY(hipMemcpy(P->d_sinst[t], P->h_sinst[t].data(), P->h_sinst[t].size(), hipMemcpyHostToDevice));
     }
     if (P->has_ir) {
@@ -2994,7 +3041,7 @@ static hss_status plan_create_impl(int32_t count, hss_fact_s* const* facts, cons
         e = dalloc(&P->d_work, work.size());
         if (e == hipSuccess) e = hipMemcpy(P->d_work, work.data(), sizeof(MvRec) * work.size(), hipMemcpyHostToDevice);
     }
-    if (e == hipSuccess) e = dalloc(&P->d_rec, P->S.rec.size());
+    if (e == hipSuccess) e = ctx->pool.get(&P->d_rec, sizeof(SweepRec) * P->S.rec.size());
     if (e == hipSuccess)
         e = hipMemcpy(P->d_rec, P->S.rec.data(), sizeof(SweepRec) * P->S.rec.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
