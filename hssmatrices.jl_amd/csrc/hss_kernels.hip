@@ -133,21 +133,6 @@ __device__ __forceinline__ T row_reduce(T v, int S) {
     return v;
 }
 
-// sum over the wave (all lanes active), as the butterfly lane ^ 1, 2, 4, 8, 16, 32: once
-// the values are equal within quads (then within half rows), the half-row mirror (then the
-// row mirror) pairs lanes exactly as ^ 4 (then ^ 8) does, so every lane ends with the same
-// sum, added in the same order
-template <typename T>
-__device__ __forceinline__ T wave_reduce(T v) {
-    v += dpp_mov<0xB1>(v);
-    v += dpp_mov<0x4E>(v);
-    v += dpp_mov<0x141>(v);
-    v += dpp_mov<0x140>(v);
-    v += shfl_xor(v, 16);
-    v += shfl_xor(v, 32);
-    return v;
-}
-
 // Sum over the four 16-lane rows of a wave (lanes l, l^16, l^32, l^48), on the VALU:
 // v_permlane16_swap then v_permlane32_swap (gfx950), each adding the value the swap brings
 // to the lane's own; every lane ends with the same sum, added in the same order.
@@ -177,6 +162,18 @@ __device__ __forceinline__ double rows_sum(double v) {
     v = pair(a[0], c[0]) + pair(a[1], c[1]);
 #endif
     return v;
+}
+// sum over the wave (all lanes active), as the butterfly lane ^ 1, 2, 4, 8, 16, 32: once
+// the values are equal within quads (then within half rows), the half-row mirror (then the
+// row mirror) pairs lanes exactly as ^ 4 (then ^ 8) does, so every lane ends with the same
+// sum, added in the same order
+template <typename T>
+__device__ __forceinline__ T wave_reduce(T v) {
+    v += dpp_mov<0xB1>(v);
+    v += dpp_mov<0x4E>(v);
+    v += dpp_mov<0x141>(v);
+    v += dpp_mov<0x140>(v);
+    return rows_sum(v);
 }
 // lane l's value (l uniform across the wave) to every lane (v_readlane)
 __device__ __forceinline__ float lane_read(float v, int l) {
@@ -414,6 +411,43 @@ __device__ ChildRed<T> child_red(const FInst<T>& I, int c) {
     return r;
 }
 
+// st(i, j, v) for v = sum_l fa(i, l) fb(l, j), i < M, j < N, the workgroup's waves sharing the
+// 16 x 16 output tiles (every thread calls; tiles counts the tiles of the calls so far, so
+// that successive products continue on the next wave).  Operands come straight from memory:
+// 48 terms of a tile are loaded at once, indices clamped so that no load is guarded.
+template <typename T, typename FA, typename FB, typename ST>
+__device__ __forceinline__ void wave_tiles(int& tiles, int M, int N, int K, FA fa, FB fb, ST st) {
+    using MF = Mfma<T>;
+    constexpr int KS = 12;
+    const int nw = blockDim.x / 64, wave = threadIdx.x >> 6, li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+    const int tm = (M + 15) / 16, count = tm * ((N + 15) / 16);
+    for (int t = (wave + nw - tiles % nw) % nw; t < count; t += nw) {
+        const int i = 16 * (t % tm) + li, j = 16 * (t / tm) + li;
+        const int ic = min(i, M - 1), jc = min(j, N - 1);
+        typename MF::v4 acc = {T(0), T(0), T(0), T(0)};
+        for (int k0 = 0; k0 < K; k0 += 4 * KS) {
+            T a[KS], b[KS];
+#pragma unroll
+            for (int q = 0; q < KS; ++q) {
+                const int l = min(k0 + 4 * q + lk, K - 1);
+                a[q] = fa(ic, l);
+                b[q] = fb(l, jc);
+            }
+#pragma unroll
+            for (int q = 0; q < KS; ++q) {
+                const bool on = k0 + 4 * q + lk < K;
+                acc = MF::mac(on ? a[q] : T(0), on ? b[q] : T(0), acc);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int io = 16 * (t % tm) + MF::row(lk, r);
+            if (io < M && j < N) st(io, j, acc[r]);
+        }
+    }
+    tiles += count;
+}
+
 // Merged diagonal block entry (r, c) of a branch node (ulvfactor.jl:75):
 //   [ D1            U1 B12 V2' ]
 //   [ U2 B21 V1'    D2         ]
@@ -462,20 +496,23 @@ __device__ __forceinline__ int vpad(int c) { return c + (c / CPT) * 2; }
 // U in LDS and the source of W = [D; V'] (phase 0), the exit of a pass-through node, the QL
 // of U with its outputs (phase 1), and M = T (Y' D) in LDS (phase 2), so that
 // Q_ql' D = D - Y M.  LDS: Us (m x ku) | G (k x k) | Tq (k x k) | M (k rows of vstride) |
-// vb (2 x vstride) | taus | sc, with vstride = S (CPT + 2) + 2.  Wm is set to the
+// vb (2 x vstride) | taus, with vstride = S (CPT + 2) + 2.  Wm is set to the
 // row-major merge buffer of a branch (null at a leaf, whose D and V are read from the
 // generator blob).  Returns false for a pass-through node, whose outputs it has written.
+// Every phase is bound by latency, not by bytes or operations.  With the merge, the QL and M
+// as they are now the launches of k_ulv_factor_mf at n = 65536 (leaf 128) went from 637 to
+// 507 us (leaves), 298 to 187 us (three levels of 65-128 rows) and 172 to 122 us (five of up
+// to 64 rows).
 template <typename T, int CPT>
 __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, const FNode& f,
-                                          unsigned char* lds_raw, const T*& Wm_out, int64_t lds_elems) {
+                                          unsigned char* lds_raw, const T*& Wm_out) {
     const int m = f.m, n = f.n, k = f.k, nk = f.nk, ku = nd.ku, kv = nd.kv;
     const int S = f.S;
     const int tid = threadIdx.x;
-    const int R = m + kv;
     const int wave = tid / 64, lane = tid % 64;
     const int nwaves = blockDim.x / 64;
 
-    // LDS: Us (m x ku) | G (k x k) | Tq (k x k) | M (k rows of vstride) | vb (2 x vstride) | taus | sc
+    // LDS: Us (m x ku) | G (k x k) | Tq (k x k) | M (k rows of vstride) | vb (2 x vstride) | taus
     // every row chunk of the S threads is CPT wide (columns >= n are zero padding)
     const int vstride = S * (CPT + 2) + 2;
     T* Us = reinterpret_cast<T*>(lds_raw);
@@ -484,7 +521,6 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
     T* Mq = Tq + (size_t)k * k;  // row j of M at Mq + j * vstride, column c at vpad(c)
     T* vbuf = Mq + (size_t)k * vstride;
     T* taus = vbuf + 2 * vstride;
-    T* sc = taus + (k > nk ? k : nk) + 1;
 
     // ---- phase 0: U (LDS); the source of W = [D; V'] ----
     //   leaf:   D and V from the generator blob (column-major)
@@ -493,146 +529,48 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
     if (nd.is_leaf) {
         for (int e = tid; e < m * ku; e += blockDim.x) Us[e] = gen<T>(I.blob, nd.U, e);
     } else {
-        const ChildRed<T> a = child_red(I, nd.left);
-        const ChildRed<T> b = child_red(I, nd.right);
-        const DevNode dl = I.nodes[nd.left];
-        const DevNode dr = I.nodes[nd.right];
+        // The merge (ulvfactor.jl:74-79) as MFMA tiles shared by the waves, in two phases: the
+        // products of generators and reduced blocks, then those with P = U1 B12 (U2 B21), which
+        // the solve operators use too.  Latency-bound (ranks of 11-35: 15-28 us a node when
+        // each product was staged in LDS between two barriers, one output a thread);
+        // the output index that is contiguous in memory runs over the lanes.
+        const FNode HSS_GLOBAL& fl = I.fn[nd.left];
         T* Wmw = I.rw + f.rwM;
-        // The merge's inner products run over the children's ranks, so they are staged:
-        // the LDS after Us (used by phases 1-5 only later) holds the rank-sized operands,
-        // loaded with many loads in flight, and the products read LDS.  The launch's
-        // dynamic LDS (lds_elems elements, at least this node's own formula) bounds what
-        // fits; a merge that does not fit reads its operands from memory.
-        const int64_t own = 2 * (int64_t)k * k + (int64_t)(k + 2) * vstride + (k > nk ? k : nk) + 1 + 8;
-        const int64_t cap = lds_elems - (int64_t)m * ku > own ? lds_elems - (int64_t)m * ku : own;
-        auto mx = [](int64_t x, int64_t y) { return x > y ? x : y; };
-        const int64_t nP12 = (int64_t)a.mr * b.kv, nP21 = (int64_t)b.mr * a.kv;
-        const int64_t nU1 = (int64_t)a.mr * a.ku, nU2 = (int64_t)b.mr * b.ku;
-        const int64_t nV1 = (int64_t)a.nr * a.kv, nV2 = (int64_t)b.nr * b.kv;
-        // the most any one step below holds at once
-        const int64_t need = mx(mx(nP12 + mx(nU1 + (int64_t)a.ku * b.kv, nV2), nP21 + mx(nU2 + (int64_t)b.ku * a.kv, nV1)),
-                                mx(mx(nV1 + (int64_t)a.kv * kv, nV2 + (int64_t)b.kv * kv),
-                                   mx(nU1 + (int64_t)a.ku * ku, nU2 + (int64_t)b.ku * ku)));
-        if (need <= cap) {
-            auto stage_to = [&](T* dst, int cnt, auto ld) { batched<8, T>(cnt, ld, [&](int e, T v) { dst[e] = v; }); };
-            // rows of the merged D (ulvfactor.jl:75): [D1, U1 B12 V2'] then [U2 B21 V1', D2].
-            // P = U1 B12 (or U2 B21) is kept in the factor too: the solve operators use it.
-            for (int half = 0; half < 2; ++half) {
-                const ChildRed<T>& x = half ? b : a;  // rows from this child
-                const ChildRed<T>& o = half ? a : b;  // the other child (columns of V')
-                const int64_t nP = (int64_t)x.mr * o.kv;
-                T* sP = G;
-                T* sU = sP + nP;
-                T* sB = sU + (int64_t)x.mr * x.ku;
-                stage_to(sU, x.mr * x.ku, [&](int e) { return x.U[e]; });
-                stage_to(sB, x.ku * o.kv, [&](int e) { return gen<T>(I.blob, half ? nd.B21 : nd.B12, e); });
-                __syncthreads();
-                T* Pg = I.tmp + (half ? f.P21 : f.P12);
-                for (int e = tid; e < nP; e += blockDim.x) {
-                    const int rr = e % x.mr, c = e / x.mr;
-                    T sum = T(0);
-                    for (int l = 0; l < x.ku; ++l) sum += sU[rr + l * x.mr] * sB[l + c * x.ku];
-                    sP[e] = sum;
-                    Pg[e] = sum;
-                }
-                __syncthreads();
-                T* sV = sU;  // the other child's V, over U and B
-                stage_to(sV, o.nr * o.kv, [&](int e) { return o.V[e]; });
-                __syncthreads();
-                const int r0 = half ? a.mr : 0, own0 = half ? a.nr : 0;  // own columns start
-                for (int e = tid; e < x.mr * n; e += blockDim.x) {
-                    const int rr = e / n, c = e % n;
-                    T val = T(0);
-                    if (c >= own0 && c < own0 + x.nr) {
-                        val = x.D[rr + (int64_t)(c - own0) * x.mr];
-                    } else {
-                        const int cc = half ? c : c - a.nr;  // column of the other child's V'
-                        for (int l = 0; l < o.kv; ++l) val += sP[rr + l * x.mr] * sV[cc + l * o.nr];
-                    }
-                    Wmw[(int64_t)(r0 + rr) * n + c] = val;
-                }
-                __syncthreads();
-            }
-            // rows of V' (ulvfactor.jl:79): V = [V1 W1; V2 W2]; columns from each child in turn
-            for (int half = 0; half < 2; ++half) {
-                const ChildRed<T>& x = half ? b : a;
-                T* sV = G;
-                T* sW = sV + (int64_t)x.nr * x.kv;
-                stage_to(sV, x.nr * x.kv, [&](int e) { return x.V[e]; });
-                stage_to(sW, x.kv * kv, [&](int e) { return gen<T>(I.blob, half ? dr.W : dl.W, e); });
-                __syncthreads();
-                const int c0x = half ? a.nr : 0;
-                for (int e = tid; e < kv * x.nr; e += blockDim.x) {
-                    const int j = e / x.nr, c = e % x.nr;
-                    T val = T(0);
-                    for (int l = 0; l < x.kv; ++l) val += sV[c + l * x.nr] * sW[l + j * x.kv];
-                    Wmw[(int64_t)(m + j) * n + c0x + c] = val;
-                }
-                __syncthreads();
-            }
+        int tiles = 0;
+        for (int h = 0; h < 2; ++h) {
+            const ChildRed<T> c = child_red(I, h ? nd.right : nd.left), o = child_red(I, h ? nd.left : nd.right);
+            const DevNode HSS_GLOBAL& dc = I.nodes[h ? nd.right : nd.left];
+            const int64_t oB = h ? nd.B21 : nd.B12, oW = dc.W, oR = dc.R;
+            T* Pg = I.tmp + (h ? f.P21 : f.P12);
+            wave_tiles<T>(tiles, o.kv, c.mr, c.ku, [&](int i, int l) { return gen<T>(I.blob, oB, l + (int64_t)i * c.ku); },
+                          [&](int l, int j) { return c.U[j + (int64_t)l * c.mr]; },
+                          [&](int i, int j, T v) { Pg[j + (int64_t)i * c.mr] = v; });
+            const int c0 = h ? fl.nr : 0, r0 = h ? fl.mr : 0;
+            // V = [V1 W1; V2 W2]  (ulvfactor.jl:79), rows of V'
+            wave_tiles<T>(tiles, kv, c.nr, c.kv, [&](int i, int l) { return gen<T>(I.blob, oW, l + (int64_t)i * c.kv); },
+                          [&](int l, int j) { return c.V[j + (int64_t)l * c.nr]; },
+                          [&](int i, int j, T v) { Wmw[(int64_t)(m + i) * n + c0 + j] = v; });
             // U = [U1 R1; U2 R2]  (ulvfactor.jl:78)
-            for (int half = 0; half < 2; ++half) {
-                const ChildRed<T>& x = half ? b : a;
-                T* sU = G;
-                T* sR = sU + (int64_t)x.mr * x.ku;
-                stage_to(sU, x.mr * x.ku, [&](int e) { return x.U[e]; });
-                stage_to(sR, x.ku * ku, [&](int e) { return gen<T>(I.blob, half ? dr.R : dl.R, e); });
-                __syncthreads();
-                const int r0 = half ? a.mr : 0;
-                for (int e = tid; e < x.mr * ku; e += blockDim.x) {
-                    const int rr = e % x.mr, j = e / x.mr;
-                    T sum = T(0);
-                    for (int l = 0; l < x.ku; ++l) sum += sU[rr + l * x.mr] * sR[l + j * x.ku];
-                    Us[(r0 + rr) + (int64_t)j * m] = sum;
-                }
-                __syncthreads();
-            }
-            Wm = Wmw;
-            __threadfence_block();
-        } else {
-            T* P12 = I.tmp + f.P12;
-            T* P21 = I.tmp + f.P21;
-            merge_products(I, nd, a, b, P12, P21);
-            __threadfence_block();
-            __syncthreads();
-            for (int e = tid; e < R * n; e += blockDim.x) {
-                const int rr = e / n, c = e % n;
-                T val;
-                if (rr < m) {
-                    val = merged_D(a, b, P12, P21, rr, c);
-                } else {
-                    // V = [V1 W1; V2 W2]  (ulvfactor.jl:79), row j of V'
-                    const int j = rr - m;
-                    T sum = T(0);
-                    if (c < a.nr) {
-                        for (int l = 0; l < a.kv; ++l)
-                            sum += a.V[c + (int64_t)l * a.nr] * gen<T>(I.blob, dl.W, l + (int64_t)j * a.kv);
-                    } else {
-                        const int cc = c - a.nr;
-                        for (int l = 0; l < b.kv; ++l)
-                            sum += b.V[cc + (int64_t)l * b.nr] * gen<T>(I.blob, dr.W, l + (int64_t)j * b.kv);
-                    }
-                    val = sum;
-                }
-                Wmw[e] = val;
-            }
-            // U = [U1 R1; U2 R2]  (ulvfactor.jl:78)
-            for (int e = tid; e < m * ku; e += blockDim.x) {
-                const int rr = e % m, j = e / m;
-                T sum = T(0);
-                if (rr < a.mr) {
-                    for (int l = 0; l < a.ku; ++l)
-                        sum += a.U[rr + (int64_t)l * a.mr] * gen<T>(I.blob, dl.R, l + (int64_t)j * a.ku);
-                } else {
-                    const int r2 = rr - a.mr;
-                    for (int l = 0; l < b.ku; ++l)
-                        sum += b.U[r2 + (int64_t)l * b.mr] * gen<T>(I.blob, dr.R, l + (int64_t)j * b.ku);
-                }
-                Us[e] = sum;
-            }
-            Wm = Wmw;
-            __threadfence_block();
+            wave_tiles<T>(tiles, ku, c.mr, c.ku, [&](int i, int l) { return gen<T>(I.blob, oR, l + (int64_t)i * c.ku); },
+                          [&](int l, int j) { return c.U[j + (int64_t)l * c.mr]; },
+                          [&](int i, int j, T v) { Us[r0 + j + (int64_t)i * m] = v; });
+            // the child's own block of the merged D (ulvfactor.jl:75)
+            batched<4, T>(c.mr * c.nr, [&](int e) { return c.D[e]; },
+                          [&](int e, T v) { Wmw[(int64_t)(r0 + e % c.mr) * n + c0 + e / c.mr] = v; });
         }
+        __threadfence_block();
+        __syncthreads();
+        // its other blocks: U1 B12 V2' and U2 B21 V1'
+        for (int h = 0; h < 2; ++h) {
+            const ChildRed<T> c = child_red(I, h ? nd.right : nd.left), o = child_red(I, h ? nd.left : nd.right);
+            const T* P = I.tmp + (h ? f.P21 : f.P12);
+            const int c0 = h ? 0 : fl.nr, r0 = h ? fl.mr : 0;
+            wave_tiles<T>(tiles, c.mr, o.nr, o.kv, [&](int i, int l) { return P[i + (int64_t)l * c.mr]; },
+                          [&](int l, int j) { return o.V[j + (int64_t)l * o.nr]; },
+                          [&](int i, int j, T v) { Wmw[(int64_t)(r0 + i) * n + c0 + j] = v; });
+        }
+        Wm = Wmw;
+        __threadfence_block();
     }
     __syncthreads();
     // entry (rr, c) of W = [D; V']
@@ -653,60 +591,78 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
     }
 
     // ---- phase 1: QL of U (m x k) in LDS, LAPACK dgeqlf semantics (ulvfactor.jl:39) ----
-    // Two barriers per reflector.  While reflector jj is applied its vector stays unscaled in
-    // LDS and each use forms col[i] * scale, the value dgeqlf stores; the stored vector is
-    // scaled in place during the next reflector's norm (another column).  beta goes to col[p]
-    // at once: the update never reads it (the vector's unit entry is implicit).  The scalars
-    // alternate between sc[0..2] and sc[4..6], so the deferred scaling reads the previous
-    // reflector's while the current one's are written.
-    for (int jj = k - 1; jj >= 0; --jj) {
-        const int p = m - k + jj;
-        T* col = Us + (int64_t)jj * m;
-        T* scj = sc + 4 * (jj & 1);
-        if (wave == 0) {
-            T part = T(0);
-            for (int i = lane; i < p; i += 64) part += col[i] * col[i];
-            part = wave_reduce(part);
-            if (lane == 0) {
-                T beta, tau, scale;
-                larfg(col[p], part, beta, tau, scale);
-                scj[0] = beta;
-                scj[1] = tau;
-                scj[2] = scale;
-                taus[jj] = tau;
-                col[p] = beta;
+    // One barrier per reflector: every wave forms the reflector for itself, its column's norm
+    // in the same reduction as the dots with the wave's own first columns (the scale 1 / (alpha
+    // - beta) multiplies the finished dot), then updates its columns.  Column jj stays as it
+    // is until all have read it: its owner keeps it in registers and stores the scaled vector
+    // after the barrier, while the others work on column jj - 1.  The chain of k reductions
+    // and barriers bounds it (0.75 us a reflector with two barriers and one wave's norm).
+    {
+        constexpr int XR = 4, CW = 4;  // rows of a lane (m <= 256), columns of a wave at once
+        for (int jj = k - 1; jj >= 0; --jj) {
+            const int p = m - k + jj;
+            T* col = Us + (int64_t)jj * m;
+            T xc[XR], norm = T(0);
+#pragma unroll
+            for (int q = 0; q < XR; ++q) {
+                xc[q] = lane + 64 * q < p ? col[lane + 64 * q] : T(0);
+                norm += xc[q] * xc[q];
+            }
+            const T alpha = col[p];
+            T beta = alpha, tau = T(0), scale = T(0);
+            bool first = true;
+            for (int cb = wave; cb < jj || first; cb += CW * nwaves) {
+                T u[CW][XR], up[CW], dot[CW];
+#pragma unroll
+                for (int w = 0; w < CW; ++w) {
+                    const int c = cb + w * nwaves;
+                    const T* uc = Us + (int64_t)c * m;
+                    dot[w] = T(0);
+                    up[w] = c < jj ? uc[p] : T(0);
+#pragma unroll
+                    for (int q = 0; q < XR; ++q) {
+                        u[w][q] = c < jj && lane + 64 * q < p ? uc[lane + 64 * q] : T(0);
+                        dot[w] += xc[q] * u[w][q];
+                    }
+                }
+#pragma unroll
+                for (int w = 0; w < CW; ++w) dot[w] = wave_reduce(dot[w]);
+                if (first) {
+                    larfg(alpha, wave_reduce(norm), beta, tau, scale);
+                    first = false;
+                }
+#pragma unroll
+                for (int w = 0; w < CW; ++w) {
+                    const int c = cb + w * nwaves;
+                    T* uc = Us + (int64_t)c * m;
+                    if (c < jj && tau != T(0)) {
+                        const T t = tau * (up[w] + scale * dot[w]), ts = t * scale;
+#pragma unroll
+                        for (int q = 0; q < XR; ++q)
+                            if (lane + 64 * q < p) uc[lane + 64 * q] = u[w][q] - ts * xc[q];
+                        if (lane == 0) uc[p] = up[w] - t;
+                    }
+                }
+            }
+            __syncthreads();
+            if (wave == jj % nwaves) {
+#pragma unroll
+                for (int q = 0; q < XR; ++q)
+                    if (lane + 64 * q < p) col[lane + 64 * q] = tau != T(0) ? xc[q] * scale : xc[q];
+                if (lane == 0) {
+                    col[p] = beta;
+                    taus[jj] = tau;
+                }
             }
         }
-        if (jj + 1 < k) {  // reflector jj + 1's vector: rows [0, p + 1) of the next column
-            const T* scp = sc + 4 * ((jj + 1) & 1);
-            if (scp[1] != T(0))
-                for (int i = tid; i < p + 1; i += blockDim.x) col[m + i] *= scp[2];
-        }
-        __syncthreads();
-        // apply H = I - tau v v' to U[0:p+1, 0:jj], v = [col[0:p] * scale; 1]
-        const T tau = scj[1], scale = scj[2];
-        if (tau != T(0)) {
-            for (int c = wave; c < jj; c += nwaves) {
-                T* uc = Us + (int64_t)c * m;
-                T part = T(0);
-                for (int i = lane; i < p; i += 64) part += (col[i] * scale) * uc[i];
-                part = wave_reduce(part) + uc[p];
-                const T t = tau * part;
-                for (int i = lane; i < p; i += 64) uc[i] -= t * (col[i] * scale);
-                if (lane == 0) uc[p] -= t;
-            }
-        }
-        __syncthreads();
-    }
-    if (k > 0) {  // reflector 0's vector: rows [0, m - k) of column 0
-        if (sc[1] != T(0))
-            for (int i = tid; i < m - k; i += blockDim.x) Us[i] *= sc[2];
         __syncthreads();
     }
     // reflector j: y_j[i] = Us[i, j] (i < p_j), 1 (i = p_j), 0 below
+    // (the load is in range for every i < m, j < k, and not guarded)
     auto yql = [&](int i, int j) -> T {
         const int p = m - k + j;
-        return i < p ? Us[i + (int64_t)j * m] : (i == p ? T(1) : T(0));
+        const T u = Us[i + j * m];
+        return i < p ? u : (i == p ? T(1) : T(0));
     };
     {
         T* Y = I.tmp + f.Yql;
@@ -716,87 +672,101 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
             const int i = e % k, j = e / k;
             Ur[e] = (i >= j) ? Us[(m - k + i) + (int64_t)j * m] : T(0);
         }
-        // Gram G[a][b] = y_a . y_b for a < b (y_a has its unit above y_b's)
-        for (int e = tid; e < k * k; e += blockDim.x) {
-            const int a = e % k, bcol = e / k;
-            T sum = T(0);
-            if (a < bcol) {
-                const int pa = m - k + a;
-                const T* ya = Us + (int64_t)a * m;
-                const T* yb = Us + (int64_t)bcol * m;
-                sum = yb[pa];
-                for (int i = 0; i < pa; ++i) sum += ya[i] * yb[i];
-            }
-            G[e] = sum;
-        }
+        // Gram G[a][b] = y_a . y_b for a < b
+        int tiles = 0;
+        wave_tiles<T>(tiles, k, k, m, [&](int a, int l) { return yql(l, a); }, [&](int l, int b) { return yql(l, b); },
+                      [&](int a, int b, T v) { G[a + b * k] = v; });
     }
-    __syncthreads();
-    // padding columns of M (n <= c < S * CPT) must read as zero in phase 3
+    // padding columns of M (n <= c < S * CPT) must read as zero in k_ulv_factor's phase 3
     for (int e = tid; e < k * vstride; e += blockDim.x) Mq[e] = T(0);
+    __syncthreads();
     // T factor of H(1)...H(k) = I - Y T Y' (dlarft, forward columnwise); row a of T
-    // depends only on row a itself, so thread a builds it alone
-    for (int a = tid; a < k; a += blockDim.x) {
-        for (int q = 0; q < k; ++q) Tq[a + (int64_t)q * k] = T(0);
-        Tq[a + (int64_t)a * k] = taus[a];
+    // depends only on row a itself, so four lanes build it alone
+    for (int a = tid >> 2; a < k; a += blockDim.x >> 2) {
+        const int q = tid & 3;
+        T* ta = Tq + a;
+        for (int i = q; i < k; i += 4) ta[(int64_t)i * k] = i == a ? taus[a] : T(0);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         for (int i = a + 1; i < k; ++i) {
             T sum = T(0);
-            for (int bb = a; bb < i; ++bb) sum += Tq[a + (int64_t)bb * k] * G[bb + (int64_t)i * k];
-            Tq[a + (int64_t)i * k] = -taus[i] * sum;
+            for (int bb = a + q; bb < i; bb += 4) sum += ta[(int64_t)bb * k] * G[bb + (int64_t)i * k];
+            sum = row_reduce(sum, 4);
+            if (q == 0) ta[(int64_t)i * k] = -taus[i] * sum;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
     }
-    __syncthreads();
-    {
-        T* Tg = I.tmp + f.Tql;
-        for (int e = tid; e < k * k; e += blockDim.x) Tg[e] = Tq[e];
-    }
-
     // ---- phase 2: M = T (Y' D), so that Q_ql' D = D - Y M  (ulvfactor.jl:41) ----
-    // thread (column c, row group g): rows g, g+16, ... ; reduction over the 16 lanes of g
+    // A wave takes 16 columns of D through both products on MFMA: Y' D (four tiles of
+    // reflectors at a time, 64 rows of D in flight, lane lk taking four adjacent rows) into M,
+    // then T times it.  Bound by the MFMA chain (96 for 128 x 128 and rank 35) and one trip to
+    // memory; a dot product a thread with lane shuffles took 14-47 us a node.
     {
-        constexpr int RG = 16, MAXR = 16;
-        const int g = tid % RG;
-        const int cols_per_pass = blockDim.x / RG;
-        for (int cb = tid / RG; cb < ((n + cols_per_pass - 1) / cols_per_pass) * cols_per_pass; cb += cols_per_pass) {
-            const int c = cb;
-            T d[MAXR];
+        using MF = Mfma<T>;
+        using V4 = typename MF::v4;
+        const int li = lane & 15, lk = lane >> 4, kt = (k + 15) / 16;
+        auto yt = [&](int c0, int q0) {  // Y' D for one column tile and reflector tiles q0 .. q0 + 3
+            const int c = c0 + li, cc = min(c, n - 1);
+            V4 acc[4];
 #pragma unroll
-            for (int q = 0; q < MAXR; ++q) {
-                const int i = g + RG * q;
-                d[q] = (c < n && i < m) ? Wsrc(i, c) : T(0);
-            }
-            for (int j0 = 0; j0 < k; j0 += 8) {
-                T acc[8];
+            for (int q = 0; q < 4; ++q) acc[q] = V4{T(0), T(0), T(0), T(0)};
+            for (int i0 = 0; i0 < m; i0 += 64) {
+                T d[16];
 #pragma unroll
-                for (int t = 0; t < 8; ++t) acc[t] = T(0);
+                for (int e = 0; e < 16; ++e) {
+                    const int i = i0 + 16 * (e >> 2) + 4 * lk + (e & 3);
+                    const T v = Wsrc(min(i, m - 1), cc);
+                    d[e] = i < m && c < n ? v : T(0);
+                }
 #pragma unroll
-                for (int q = 0; q < MAXR; ++q) {
-                    const int i = g + RG * q;
-                    if (i < m) {
+                for (int q = 0; q < 4; ++q) {
+                    if (q0 + q >= kt) continue;
+                    const int j = 16 * (q0 + q) + li, jc = min(j, k - 1);
 #pragma unroll
-                        for (int t = 0; t < 8; ++t)
-                            if (j0 + t < k) acc[t] += yql(i, j0 + t) * d[q];
+                    for (int e = 0; e < 16; ++e) {
+                        const int i = i0 + 16 * (e >> 2) + 4 * lk + (e & 3);
+                        const T y = yql(min(i, m - 1), jc);
+                        acc[q] = MF::mac(i < m && j < k ? y : T(0), d[e], acc[q]);
                     }
                 }
+            }
 #pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    T v = acc[t];
-                    v += shfl_xor(v, 1);
-                    v += shfl_xor(v, 2);
-                    v += shfl_xor(v, 4);
-                    v += shfl_xor(v, 8);
-                    if (g == 0 && c < n && j0 + t < k) Mq[(j0 + t) * vstride + vpad<CPT>(c)] = v;
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int j = 16 * (q0 + q) + MF::row(lk, r);
+                    if (j < k && c < n) Mq[j * vstride + vpad<CPT>(c)] = acc[q][r];
+                }
+        };
+        for (int c0 = 16 * wave; c0 < n; c0 += 16 * nwaves)
+            for (int q0 = 0; q0 < kt; q0 += 4) yt(c0, q0);
+        __syncthreads();  // T
+        {
+            T* Tg = I.tmp + f.Tql;
+            for (int e = tid; e < k * k; e += blockDim.x) Tg[e] = Tq[e];
+        }
+        // M <- T M in place, the wave's own columns (T upper triangular: ascending tiles read
+        // only rows at and below their own)
+        for (int c0 = 16 * wave; c0 < n; c0 += 16 * nwaves) {
+            const int c = c0 + li;
+            const T* mc = Mq + vpad<CPT>(min(c, n - 1));
+            for (int q = 0; q < kt; ++q) {
+                V4 acc = {T(0), T(0), T(0), T(0)};
+                const int j = 16 * q + li;
+                for (int t = q; t < kt; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int l = 16 * t + 4 * r + lk;
+                        const T tv = Tq[min(j, k - 1) + (int64_t)min(l, k - 1) * k], mv = mc[min(l, k - 1) * vstride];
+                        acc = MF::mac(j < k && l < k ? tv : T(0), c < n && l < k ? mv : T(0), acc);
+                    }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int jo = 16 * q + MF::row(lk, r);
+                    if (jo < k && c < n) Mq[jo * vstride + vpad<CPT>(c)] = acc[r];
                 }
             }
-        }
-    }
-    __syncthreads();
-    // M <- T M in place (T upper triangular: ascending j reads only rows >= j)
-    for (int c = tid; c < n; c += blockDim.x) {
-        T* mc = Mq + vpad<CPT>(c);
-        for (int j = 0; j < k; ++j) {
-            T sum = T(0);
-            for (int l = j; l < k; ++l) sum += Tq[j + (int64_t)l * k] * mc[l * vstride];
-            mc[j * vstride] = sum;
         }
     }
     __syncthreads();
@@ -810,7 +780,7 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
 // without spills and keeps them.
 template <typename T, int CPT, int NT>
 __global__ __launch_bounds__(NT) void k_ulv_factor(const FInst<T>* __restrict__ insts,
-                                                             const WorkItem* __restrict__ work, int64_t lds_elems) {
+                                                             const WorkItem* __restrict__ work) {
     const WorkItem wi = work[blockIdx.x];
     const FInst<T>& I = insts[wi.inst];
     const DevNode nd = I.nodes[wi.node];
@@ -824,7 +794,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor(const FInst<T>* __restrict__ 
     const bool row_on = r < R;
     extern __shared__ unsigned char lds_raw[];
     const T* Wm = nullptr;
-    if (!ulv_front<T, CPT>(I, nd, f, lds_raw, Wm, lds_elems)) return;
+    if (!ulv_front<T, CPT>(I, nd, f, lds_raw, Wm)) return;
     const int vstride = S * (CPT + 2) + 2;
     T* Us = reinterpret_cast<T*>(lds_raw);
     T* Mq = Us + (size_t)m * nd.ku + 2 * (size_t)k * k;
@@ -957,7 +927,7 @@ template <typename T>
 struct LqPanel {
     static constexpr int TPP = 17;
     static constexpr int pitch(int ntile) { return 16 * ntile + 2; }
-    T *Vs, *Ts, *tl;
+    T *Vs, *Ts;
     T* Tg;  // the factor's T blocks (global)
     int nk, wave, lane;
 };
@@ -989,7 +959,7 @@ __device__ __forceinline__ void lq_panels(typename Mfma<T>::v4 (&a)[NTILE], cons
     T* Tp = L.Ts + (P & 1) * 16 * TPP;
     if (L.wave == P) {
         T tr[4] = {T(0), T(0), T(0), T(0)};  // T(li, 4 r + lk)
-        T scale = T(0), mytau = T(0);  // of reflector li, once formed
+        T scale = T(0);                // of reflector li, once formed
         T g = T(0), ptau = T(0);       // reflector j - 1's Gram column and tau
         // T(li, j) = -tau_j sum_{li <= b < j} T(li, b) (v_b . v_j) for li < j (g is zero
         // from lane j on)
@@ -1049,7 +1019,6 @@ __device__ __forceinline__ void lq_panels(typename Mfma<T>::v4 (&a)[NTILE], cons
             g = li < j ? scale * d : T(0);
             ptau = tau;
             scale = own ? scl : scale;
-            mytau = own ? tau : mytau;
         }
         tcol(nb - 1);
         // the reflectors scaled, in the rows and (columns in order, rows beyond nb zero) in
@@ -1070,7 +1039,6 @@ __device__ __forceinline__ void lq_panels(typename Mfma<T>::v4 (&a)[NTILE], cons
             Tp[li * TPP + 4 * r + lk] = x;
             Tg[li + (4 * r + lk) * NB] = x;
         }
-        if (lk == 0 && li < nb) L.tl[i0 + li] = mytau;
     }
     __syncthreads();
     if (L.wave > P) {
@@ -1105,11 +1073,13 @@ __device__ __forceinline__ void lq_panels(typename Mfma<T>::v4 (&a)[NTILE], cons
 //   forms their compact-WY T (dlarft forward, from the Gram V V' on MFMA); then every wave
 //   below applies the block, W <- W (I - V' T V) = W - ((W V') T) V, as three MFMA chains.
 //   One workgroup barrier per panel (V and T double-buffered).
-// Outputs as k_ulv_factor (L1, the LQ reflectors, L2a, V_top, the reduced D and V, taus)
+// Outputs as k_ulv_factor (L1, the LQ reflectors, L2a, V_top, the reduced D and V)
 // plus the T blocks and the inverted diagonal blocks of L1 (k_ulv_wy's outputs).
+// NTILE = 4 is held to four waves per SIMD, so that two workgroups share a CU on the batched
+// levels (one costs them 30 %).
 template <typename T, int NTILE, int NT>
-__global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict__ insts,
-                                                      const WorkItem* __restrict__ work, int64_t lds_elems) {
+__global__ __launch_bounds__(NT, NT == 512 && NTILE == 4 ? 4 : 1) void k_ulv_factor_mf(const FInst<T>* __restrict__ insts,
+                                                      const WorkItem* __restrict__ work) {
     using MF = Mfma<T>;
     using V4 = typename MF::v4;
     constexpr int NC = 16 * NTILE;  // columns held per row (n <= NC)
@@ -1119,7 +1089,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
     const FNode f = I.fn[wi.node];
     extern __shared__ unsigned char lds_raw[];
     const T* Wm = nullptr;
-    if (!ulv_front<T, FACT_CPT>(I, nd, f, lds_raw, Wm, lds_elems)) return;
+    if (!ulv_front<T, FACT_CPT>(I, nd, f, lds_raw, Wm)) return;
     const int m = f.m, n = f.n, k = f.k, nk = f.nk, kv = nd.kv, R = m + kv;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, lk = lane >> 4;
@@ -1135,13 +1105,11 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
     for (int t = 0; t < NTILE; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int c = colof(t, r);
-            T x = T(0);
-            if (row < R && c < n) {
-                if (Wm) x = Wm[(int64_t)row * n + c];
-                else x = row < m ? gen<T>(I.blob, nd.D, row + (int64_t)c * m) : gen<T>(I.blob, nd.V, c + (int64_t)(row - m) * n);
-            }
-            a[t][r] = x;
+            const int c = colof(t, r), rc = min(row, R - 1), cc = min(c, n - 1);
+            T x;
+            if (Wm) x = Wm[(int64_t)rc * n + cc];
+            else x = (T)I.blob[rc < m ? nd.D + rc + (int64_t)cc * m : nd.V + cc + (int64_t)(rc - m) * n];
+            a[t][r] = row < R && c < n ? x : T(0);
         }
     for (int s4 = 0; s4 < (k + 3) / 4; ++s4) {
         const int kk = 4 * s4 + lk;  // the k index this lane supplies in the step
@@ -1169,8 +1137,7 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
     // distinct LDS banks
     constexpr int TPP = LqPanel<T>::TPP;
     T* Ts = Vs + 2 * 16 * NCP;
-    T* tl = Ts + 2 * 16 * TPP;              // nk taus (nk <= n <= 128)
-    lq_panels<T, NTILE, 0>(a, LqPanel<T>{Vs, Ts, tl, I.tmp + f.Tlq, nk, wave, lane});
+    lq_panels<T, NTILE, 0>(a, LqPanel<T>{Vs, Ts, I.tmp + f.Tlq, nk, wave, lane});
     // Inverse of L1's diagonal block `wave`, which this wave holds: lane li solves L x = e_li.
     // (A kernel of its own after the factor, which also formed T again, took 245 us on 1022
     // nodes, one wave a block and its operands from memory.)
@@ -1195,7 +1162,6 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
             for (int q = 0; q < 16; ++q) Lig[q + li * NB] = x[q];
         }
     }
-    __syncthreads();
 
     // ---- outputs (the same blocks and layouts as k_ulv_factor's phase 5) ----
     // (the row index passes through an empty asm so that the output addresses are formed
@@ -1225,7 +1191,6 @@ __global__ __launch_bounds__(NT) void k_ulv_factor_mf(const FInst<T>* __restrict
                 }
             }
     }
-    for (int e = tid; e < nk; e += blockDim.x) I.tmp[f.taulq + e] = tl[e];
 }
 
 // Compact-WY T blocks of the LQ reflectors (dlarft, forward columnwise) and the
@@ -1595,9 +1560,9 @@ __device__ __forceinline__ typename Mfma<TF>::v4 tile_mac(const TF* __restrict__
     const int i = i0 + li;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int kk = k0 + Mfma<TF>::row(lk, r);
-        TF v = TF(0);
-        if (i < M && kk < K) v = TA ? A[kk + (int64_t)i * lda] : A[i + (int64_t)kk * lda];
+        const int kk = k0 + Mfma<TF>::row(lk, r), ic = min(i, M - 1), kc = min(kk, K - 1);
+        TF v = TA ? A[kc + (int64_t)ic * lda] : A[ic + (int64_t)kc * lda];  // clamped, so not guarded
+        v = i < M && kk < K ? v : TF(0);
         acc = Mfma<TF>::mac(neg ? -v : v, x[r], acc);
     }
     return acc;
@@ -3017,7 +2982,7 @@ static hipError_t launch_factor_nt(const FInst<T>* insts, const WorkItem* work, 
     const void* fn = reinterpret_cast<const void*>(&k_ulv_factor<T, FACT_CPT, NT>);
     hipError_t e = set_lds_attr<T>(fn, lds);
     if (e != hipSuccess) return e;
-    klaunch((k_ulv_factor<T, FACT_CPT, NT>), dim3(nwork), dim3(NT), lds, st, insts, work, (int64_t)(lds / sizeof(T)));
+    klaunch((k_ulv_factor<T, FACT_CPT, NT>), dim3(nwork), dim3(NT), lds, st, insts, work);
     return hipGetLastError();
 }
 template <typename T, int NTILE, int NT>
@@ -3026,7 +2991,7 @@ static hipError_t launch_factor_mf_nt(const FInst<T>* insts, const WorkItem* wor
     const void* fn = reinterpret_cast<const void*>(&k_ulv_factor_mf<T, NTILE, NT>);
     hipError_t e = set_lds_attr<T>(fn, lds);
     if (e != hipSuccess) return e;
-    klaunch((k_ulv_factor_mf<T, NTILE, NT>), dim3(nwork), dim3(NT), lds, st, insts, work, (int64_t)(lds / sizeof(T)));
+    klaunch((k_ulv_factor_mf<T, NTILE, NT>), dim3(nwork), dim3(NT), lds, st, insts, work);
     return hipGetLastError();
 }
 template <typename T, int NTILE>
