@@ -448,45 +448,6 @@ __device__ __forceinline__ void wave_tiles(int& tiles, int M, int N, int K, FA f
     tiles += count;
 }
 
-// Merged diagonal block entry (r, c) of a branch node (ulvfactor.jl:75):
-//   [ D1            U1 B12 V2' ]
-//   [ U2 B21 V1'    D2         ]
-// with P12 = U1 B12 and P21 = U2 B21 precomputed.
-template <typename T>
-__device__ __forceinline__ T merged_D(const ChildRed<T>& a, const ChildRed<T>& b, const T* P12, const T* P21, int r,
-                                      int c) {
-    if (r < a.mr) {
-        if (c < a.nr) return a.D[r + (int64_t)c * a.mr];
-        const int cc = c - a.nr;
-        T s = T(0);
-        for (int l = 0; l < b.kv; ++l) s += P12[r + (int64_t)l * a.mr] * b.V[cc + (int64_t)l * b.nr];
-        return s;
-    }
-    const int rr = r - a.mr;
-    if (c >= a.nr) return b.D[rr + (int64_t)(c - a.nr) * b.mr];
-    T s = T(0);
-    for (int l = 0; l < a.kv; ++l) s += P21[rr + (int64_t)l * b.mr] * a.V[c + (int64_t)l * a.nr];
-    return s;
-}
-
-// P12 = U1 B12 (mr1 x kv2), P21 = U2 B21 (mr2 x kv1) into global memory.
-template <typename T>
-__device__ void merge_products(const FInst<T>& I, const DevNode& nd, const ChildRed<T>& a, const ChildRed<T>& b, T* P12,
-                               T* P21) {
-    for (int e = threadIdx.x; e < a.mr * b.kv; e += blockDim.x) {
-        const int r = e % a.mr, c = e / a.mr;
-        T s = T(0);
-        for (int l = 0; l < a.ku; ++l) s += a.U[r + (int64_t)l * a.mr] * gen<T>(I.blob, nd.B12, l + (int64_t)c * a.ku);
-        P12[e] = s;
-    }
-    for (int e = threadIdx.x; e < b.mr * a.kv; e += blockDim.x) {
-        const int r = e % b.mr, c = e / b.mr;
-        T s = T(0);
-        for (int l = 0; l < b.ku; ++l) s += b.U[r + (int64_t)l * b.mr] * gen<T>(I.blob, nd.B21, l + (int64_t)c * b.ku);
-        P21[e] = s;
-    }
-}
-
 // Padded index of column c in the LQ reflector buffer: the CPT-column chunks of
 // the S threads of a row start in different LDS banks.
 template <int CPT>
@@ -1281,82 +1242,106 @@ __global__ __launch_bounds__(256) void k_ulv_wy(const FInst<T>* __restrict__ ins
 }
 
 // Root: merge the two children (or take the leaf D) and LU-factor with partial pivoting.
-template <typename T>
-__global__ __launch_bounds__(1024) void k_ulv_root(const FInst<T>* __restrict__ insts,
-                                                   const WorkItem* __restrict__ work) {
+// One workgroup works through m dependent steps, so it is bound by their latency: the block
+// is kept in LDS (L; odd pitch, so rows are free of bank conflicts too) where it fits, every
+// wave searches the pivot for itself, and a step has three barriers.  In memory, with four
+// barriers a step and the merge one output a thread, it took 132 us on the n = 65536 log kernel
+// (86 now), 69 us on the n = 2001 Cauchy matrix (50) and 104 us on 32 Cauchy matrices (71).
+constexpr int ROOT_THREADS = 512;
+template <typename T, bool L>
+__global__ __launch_bounds__(ROOT_THREADS) void k_ulv_root(const FInst<T>* __restrict__ insts,
+                                                           const WorkItem* __restrict__ work) {
     const WorkItem wi = work[blockIdx.x];
     const FInst<T>& I = insts[wi.inst];
     const DevNode nd = I.nodes[wi.node];
     const FNode f = I.fn[wi.node];
-    const int m = f.m;
-    T* A = I.fac + f.LU;
+    const int m = f.m, lda = L ? m | 1 : m;
+    extern __shared__ unsigned char lds_raw[];
+    T* A;
+    if constexpr (L) A = reinterpret_cast<T*>(lds_raw);
+    else A = I.fac + f.LU;
     int32_t* piv = I.ipiv + f.piv;
     const int tid = threadIdx.x;
     if (nd.is_leaf) {
-        for (int e = tid; e < m * m; e += blockDim.x) A[e] = gen<T>(I.blob, nd.D, e);
+        for (int e = tid; e < m * m; e += blockDim.x) A[e % m + e / m * lda] = gen<T>(I.blob, nd.D, e);
     } else {
-        const ChildRed<T> a = child_red(I, nd.left);
-        const ChildRed<T> b = child_red(I, nd.right);
-        T* P12 = I.fac + f.P12;
-        T* P21 = I.fac + f.P21;
-        merge_products(I, nd, a, b, P12, P21);
+        // [D1, U1 B12 V2'; U2 B21 V1', D2]  (ulvfactor.jl:75)
+        const FNode HSS_GLOBAL& fl = I.fn[nd.left];
+        int tiles = 0;
+        for (int h = 0; h < 2; ++h) {
+            const ChildRed<T> c = child_red(I, h ? nd.right : nd.left), o = child_red(I, h ? nd.left : nd.right);
+            const int64_t oB = h ? nd.B21 : nd.B12;
+            T* Pg = I.fac + (h ? f.P21 : f.P12);
+            wave_tiles<T>(tiles, o.kv, c.mr, c.ku, [&](int i, int l) { return gen<T>(I.blob, oB, l + (int64_t)i * c.ku); },
+                          [&](int l, int j) { return c.U[j + (int64_t)l * c.mr]; },
+                          [&](int i, int j, T v) { Pg[j + (int64_t)i * c.mr] = v; });
+            const int c0 = h ? fl.nr : 0, r0 = h ? fl.mr : 0;
+            batched<4, T>(c.mr * c.nr, [&](int e) { return c.D[e]; },
+                          [&](int e, T v) { A[r0 + e % c.mr + (c0 + e / c.mr) * lda] = v; });
+        }
         __threadfence_block();
         __syncthreads();
-        for (int e = tid; e < m * m; e += blockDim.x) A[e] = merged_D(a, b, P12, P21, e % m, e / m);
+        for (int h = 0; h < 2; ++h) {
+            const ChildRed<T> c = child_red(I, h ? nd.right : nd.left), o = child_red(I, h ? nd.left : nd.right);
+            const T* P = I.fac + (h ? f.P21 : f.P12);
+            const int c0 = h ? 0 : fl.nr, r0 = h ? fl.mr : 0;
+            wave_tiles<T>(tiles, c.mr, o.nr, o.kv, [&](int i, int l) { return P[i + (int64_t)l * c.mr]; },
+                          [&](int l, int j) { return o.V[j + (int64_t)l * o.nr]; },
+                          [&](int i, int j, T v) { A[r0 + i + (c0 + j) * lda] = v; });
+        }
     }
     __threadfence_block();
     __syncthreads();
     if (f.Dr >= 0)  // the merged block itself, for the refinement step of every root solve
-        for (int e = tid; e < m * m; e += blockDim.x) I.fac[f.Dr + e] = A[e];
-    __shared__ int s_piv;
-    __shared__ T s_val;
+        for (int e = tid; e < m * m; e += blockDim.x) I.fac[f.Dr + e] = A[e % m + e / m * lda];
     const int wave = tid / 64, lane = tid % 64;
     int info = 0;
     for (int i = 0; i < m; ++i) {
-        if (wave == 0) {
-            // idamax over A[i:m, i] (first index of the largest magnitude).  bi starts at
-            // i, so an all-NaN column pivots in range (and is reported below)
-            T best = T(-1);
-            int bi = i;
-            for (int rr = i + lane; rr < m; rr += 64) {
-                const T v = fabs(A[rr + (int64_t)i * m]);
-                if (v > best) { best = v; bi = rr; }
-            }
-            for (int o = 1; o < 64; o <<= 1) {
-                const T ob = __shfl_xor(best, o, 64);
-                const int oi = __shfl_xor(bi, o, 64);
-                if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
-            }
-            if (lane == 0) {
-                s_piv = bi;
-                s_val = A[bi + (int64_t)i * m];
-                piv[i] = bi;
-            }
+        // idamax over A[i:m, i] (first index of the largest magnitude).  bi starts at
+        // i, so an all-NaN column pivots in range (and is reported below)
+        T best = T(-1);
+        int p = i;
+        for (int rr = i + lane; rr < m; rr += 64) {
+            const T v = fabs(A[rr + i * lda]);
+            if (v > best) { best = v; p = rr; }
         }
-        __syncthreads();
-        const int p = s_piv;
-        const T pv = s_val;
+        for (int o = 1; o < 64; o <<= 1) {
+            const T ob = __shfl_xor(best, o, 64);
+            const int oi = __shfl_xor(p, o, 64);
+            if (ob > best || (ob == best && oi < p)) { best = ob; p = oi; }
+        }
+        const T pv = A[p + i * lda];
+        if (tid == 0) piv[i] = p;
         if (pv == T(0) || pv != pv) {  // a zero or NaN pivot: singular (status i + 1)
-            if (info == 0) info = i + 1;
-        } else {
-            if (p != i)
-                for (int c = tid; c < m; c += blockDim.x) {
-                    const T t = A[i + (int64_t)c * m];
-                    A[i + (int64_t)c * m] = A[p + (int64_t)c * m];
-                    A[p + (int64_t)c * m] = t;
+            info = i + 1;
+            break;
+        }
+        __syncthreads();  // column i is read
+        const T rcp = T(1) / pv;
+        if (p != i)
+            for (int c = tid; c < m; c += blockDim.x)
+                if (c != i) {
+                    const T t = A[i + c * lda];
+                    A[i + c * lda] = A[p + c * lda];
+                    A[p + c * lda] = t;
                 }
-            __syncthreads();
-            const T rcp = T(1) / pv;
-            for (int rr = i + 1 + tid; rr < m; rr += blockDim.x) A[rr + (int64_t)i * m] *= rcp;
+        for (int rr = i + 1 + tid; rr < m; rr += blockDim.x) {
+            T v = A[rr + i * lda];
+            if (rr == p) {  // rows i and p trade places here as well
+                v = A[i + i * lda];
+                A[i + i * lda] = pv;
+            }
+            A[rr + i * lda] = v * rcp;
         }
         __syncthreads();
-        const int mm = m - i - 1;
-        for (int e = tid; e < mm * mm; e += blockDim.x) {
-            const int rr = i + 1 + e % mm, c = i + 1 + e / mm;
-            A[rr + (int64_t)c * m] -= A[rr + (int64_t)i * m] * A[i + (int64_t)c * m];
+        for (int rr = i + 1 + lane; rr < m; rr += 64) {
+            const T l = A[rr + i * lda];
+            for (int c = i + 1 + wave; c < m; c += ROOT_THREADS / 64) A[rr + c * lda] -= l * A[i + c * lda];
         }
         __syncthreads();
     }
+    if constexpr (L)
+        for (int e = tid; e < m * m; e += blockDim.x) I.fac[f.LU + e] = A[e % m + e / m * lda];
     if (tid == 0) I.status[0] = info;
     // inverted diagonal NB x NB blocks of the unit-lower L and the upper U, for
     // blocked triangular solves in every root solve; thread (block, column j)
@@ -1376,7 +1361,7 @@ __global__ __launch_bounds__(1024) void k_ulv_root(const FInst<T>* __restrict__ 
                 T sum = (i2 == jj) ? T(1) : T(0);
 #pragma unroll
                 for (int q = 0; q < NB; ++q)
-                    if (q < i2 && i2 < nb) sum -= A[(b0 + i2) + (int64_t)(b0 + q) * m] * x[q];
+                    if (q < i2 && i2 < nb) sum -= A[(b0 + i2) + (b0 + q) * lda] * x[q];
                 x[i2] = (i2 < nb && jj < nb) ? sum : T(0);
             }
 #pragma unroll
@@ -1387,8 +1372,8 @@ __global__ __launch_bounds__(1024) void k_ulv_root(const FInst<T>* __restrict__ 
                 T sum = (i2 == jj) ? T(1) : T(0);
 #pragma unroll
                 for (int q = 0; q < NB; ++q)
-                    if (q > i2 && q < nb) sum -= A[(b0 + i2) + (int64_t)(b0 + q) * m] * x[q];
-                x[i2] = (i2 < nb && jj < nb) ? sum / A[(b0 + i2) + (int64_t)(b0 + i2) * m] : T(0);
+                    if (q > i2 && q < nb) sum -= A[(b0 + i2) + (b0 + q) * lda] * x[q];
+                x[i2] = (i2 < nb && jj < nb) ? sum / A[(b0 + i2) + (b0 + i2) * lda] : T(0);
             }
 #pragma unroll
             for (int q = 0; q < NB; ++q) Ui[(int64_t)bb * NB * NB + q + jj * NB] = x[q];
@@ -3031,9 +3016,17 @@ hipError_t launch_ulv_wy(const FInst<T>* insts, const WorkItem* work, int nwork,
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwork, hipStream_t st) {
+hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, hipStream_t st) {
     if (nwork <= 0) return hipSuccess;
-    klaunch((k_ulv_root<T>), dim3(nwork), dim3(1024), 0, st, insts, work);
+    const size_t lds = sizeof(T) * (size_t)max_m * (size_t)(max_m | 1);
+    if (lds <= 160 * 1024) {
+        const void* fn = reinterpret_cast<const void*>(&k_ulv_root<T, true>);
+        hipError_t e = set_lds_attr<T>(fn, lds);
+        if (e != hipSuccess) return e;
+        klaunch((k_ulv_root<T, true>), dim3(nwork), dim3(ROOT_THREADS), lds, st, insts, work);
+    } else {
+        klaunch((k_ulv_root<T, false>), dim3(nwork), dim3(ROOT_THREADS), 0, st, insts, work);
+    }
     return hipGetLastError();
 }
 template <typename T>
@@ -3847,8 +3840,8 @@ template hipError_t launch_ulv_factor_mf<float>(const FInst<float>*, const WorkI
                                                 hipStream_t);
 template hipError_t launch_ulv_wy<double>(const FInst<double>*, const WorkItem*, int, hipStream_t);
 template hipError_t launch_ulv_wy<float>(const FInst<float>*, const WorkItem*, int, hipStream_t);
-template hipError_t launch_ulv_root<double>(const FInst<double>*, const WorkItem*, int, hipStream_t);
-template hipError_t launch_ulv_root<float>(const FInst<float>*, const WorkItem*, int, hipStream_t);
+template hipError_t launch_ulv_root<double>(const FInst<double>*, const WorkItem*, int, int, hipStream_t);
+template hipError_t launch_ulv_root<float>(const FInst<float>*, const WorkItem*, int, int, hipStream_t);
 #define HSS_INST_SOLVE(T)                                                                                      \
     template hipError_t launch_ulv_gform<T>(const FInst<T>*, const WorkItem*, int, int, size_t, hipStream_t);       \
     template hipError_t launch_ulv_qform<T>(const FInst<T>*, const WorkItem*, int, int, size_t, hipStream_t);       \

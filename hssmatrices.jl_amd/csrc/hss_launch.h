@@ -46,7 +46,7 @@ int factor_mf_max_rows(int elem_bytes);
 template <typename T>
 hipError_t launch_ulv_wy(const FInst<T>* insts, const WorkItem* work, int nwork, hipStream_t st);
 template <typename T>
-hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwork, hipStream_t st);
+hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, hipStream_t st);
 // solve operators, once per factorization (every non-root node in one launch)
 // Gz, Gr and Qt of nodes with at most FORM_W_ROWS rows (k_ulv_gform_w, k_ulv_qform_w)
 constexpr int FORM_W_ROWS = 128;

@@ -2037,11 +2037,12 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
         if (s != HSS_OK) { cleanup(); return s; }
     }
     size_t lds_gform = 0, lds_qform = 0, lds_rinv = 0;
-    int max_rcols = 0;
+    int max_rcols = 0, max_rm = 0;
     for (auto* F : out) {
         lds_gform = std::max(lds_gform, F->lds_gform);
         lds_qform = std::max(lds_qform, F->lds_qform);
         const FNode& r = F->hfn[0];
+        max_rm = std::max(max_rm, r.m);
         if (r.Dinv >= 0) {
             max_rcols = std::max(max_rcols, std::max(r.m, r.Kx));
             lds_rinv = std::max(lds_rinv, sizeof(TF) * (size_t)(r.m + NB) * RHS_TILE);
@@ -2160,7 +2161,7 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
         }
         {
             ProfScope ps("k_ulv_root", 0, roots.count, st);
-            HIP_TRY((launch_ulv_root<TF>(d_inst, d_work + roots.off, roots.count, st)));
+            HIP_TRY((launch_ulv_root<TF>(d_inst, d_work + roots.off, roots.count, max_rm, st)));
         }
         {
             ProfScope ps("k_ulv_rinv", 0, roots.count, st);
