@@ -1387,153 +1387,6 @@ __global__ __launch_bounds__(ROOT_THREADS) void k_ulv_root(const FInst<T>* __res
 // The reduction of a node (ulvfactor.jl:42,48-51,74,89: Q_ql' b, the forward
 // substitution with L1, the reduced b and u, the children's merges) is linear in
 // its input x = the leaf's rows of B, or [b_1; u_1; b_2; u_2] for a branch.
-template <bool TA, typename TF, typename Store>
-__device__ __forceinline__ void mfma_gemm(int M, int K, const TF* __restrict__ A, int64_t lda, const TF* xs, int ncols,
-                                          Store store, int xp);
-
-// k_ulv_gform runs its steps on columns of the identity:
-//   Gz (nk x Kx):   column c = zloc for x = e_c
-//   Gr (R x (Kx + nk)), R = mr + kv: column c < Kx = [(Q_ql' b)[nk:m]; W_1'u_1 + W_2'u_2]
-//                   for x = e_c (the reduced b and u before their zloc terms); the last
-//                   nk columns are [-L2a; V_top'], so [reduced b; u] = Gr [x; zloc].
-// Grid columns run over Kx + nk; the last nk are copies of factor blocks.
-//
-// LDS (row-major, NTP columns): bv m rows | zl max(nk,1) | us kv_1 + kv_2 | t1 tr | t2 tr,
-// tr = max(k, NB, kv)
-template <typename TF>
-__global__ __launch_bounds__(SWEEP_THREADS) void k_ulv_gform(const FInst<TF>* __restrict__ insts,
-                                                            const WorkItem* __restrict__ work) {
-    const WorkItem wi = work[blockIdx.x];
-    const FInst<TF>& I = insts[wi.inst];
-    const DevNode nd = I.nodes[wi.node];
-    const FNode f = I.fn[wi.node];
-    const int j0 = blockIdx.y * RHS_TILE;
-    const int Kx = f.Kx, nk = f.nk, mr = f.mr, kv = nd.kv, R = mr + kv;
-    if (j0 >= Kx + nk) return;
-    TF* Gr = I.fac + f.Gr;  // ld R
-    // columns [Kx, Kx + nk) of Gr: [-L2a; V_top']
-    for (int c = max(j0, Kx); c < min(j0 + RHS_TILE, Kx + nk); ++c) {
-        const int l = c - Kx;
-        for (int i = threadIdx.x; i < R; i += blockDim.x)
-            Gr[i + (int64_t)c * R] = i < mr ? -I.tmp[f.L2a + i + (int64_t)l * f.k] : I.tmp[f.Vt + l + (int64_t)(i - mr) * nk];
-    }
-    if (j0 >= Kx) return;
-    const int nt = min(RHS_TILE, Kx - j0);
-    const int m = f.m, k = f.k;
-    int kvl = 0, kvr = 0, mrl = 0;
-    if (!nd.is_leaf) {
-        kvl = I.nodes[nd.left].kv;
-        kvr = I.nodes[nd.right].kv;
-        mrl = I.fn[nd.left].mr;
-    }
-    const int tr = max(max(k, NB), kv);
-    extern __shared__ unsigned char lds_raw[];
-    TF* bv = reinterpret_cast<TF*>(lds_raw);
-    TF* zl = bv + m * NTP;
-    TF* us = zl + max(nk, 1) * NTP;
-    TF* t1 = us + (kvl + kvr) * NTP;
-    TF* t2 = t1 + tr * NTP;
-    // identity columns j0.. scattered over b (bv) and the children's u (us):
-    // input index of bv row r is r (b_1) or r + kv_1 (b_2); of us row r, mr_1 + r (u_1) or m + r (u_2)
-    for (int e = threadIdx.x; e < m * NTP; e += blockDim.x) {
-        const int r = e / NTP, j = e % NTP;
-        const int c = (nd.is_leaf || r < mrl) ? r : r + kvl;
-        bv[e] = (j < nt && c == j0 + j) ? TF(1) : TF(0);
-    }
-    for (int e = threadIdx.x; e < (kvl + kvr) * NTP; e += blockDim.x) {
-        const int r = e / NTP, j = e % NTP;
-        const int c = r < kvl ? mrl + r : m + r;
-        us[e] = (j < nt && c == j0 + j) ? TF(1) : TF(0);
-    }
-    __syncthreads();
-    if (!nd.is_leaf) {
-        // b = [b_1 - P12 u_2; b_2 - P21 u_1]   (ulvfactor.jl:74)
-        const int mrr = m - mrl;
-        mfma_gemm<false, TF>(mrl, kvr, I.tmp + f.P12, mrl, us + kvl * NTP, nt,
-                         [&](int i, int j, TF v) { bv[i * NTP + j] -= v; }, NTP);
-        mfma_gemm<false, TF>(mrr, kvl, I.tmp + f.P21, mrr, us, nt,
-                         [&](int i, int j, TF v) { bv[(mrl + i) * NTP + j] -= v; }, NTP);
-        __syncthreads();
-    }
-    TF* Grc = Gr + (int64_t)j0 * R;  // column j0 of Gr
-    if (!f.pass) {
-        // b <- Q_ql' b = b - Y (T (Y' b))   (ulvfactor.jl:42)
-        if (k > 0) {
-            mfma_gemm<true, TF>(k, m, I.tmp + f.Yql, m, bv, nt, [&](int i, int j, TF v) { t1[i * NTP + j] = v; }, NTP);
-            __syncthreads();
-            mfma_gemm<false, TF>(k, k, I.tmp + f.Tql, k, t1, nt, [&](int i, int j, TF v) { t2[i * NTP + j] = v; }, NTP);
-            __syncthreads();
-            mfma_gemm<false, TF>(m, k, I.tmp + f.Yql, m, t2, nt, [&](int i, int j, TF v) { bv[i * NTP + j] -= v; }, NTP);
-            __syncthreads();
-        }
-        // zloc = L1 \ b[0:nk]  (ulvfactor.jl:48), blocked with inverted diagonal blocks
-        for (int bb = 0; bb < f.nblk; ++bb) {
-            const int b0 = bb * NB, nb = min(NB, nk - b0);
-            mfma_gemm<false, TF>(nb, b0, I.tmp + f.L1 + b0, nk, zl, nt,
-                             [&](int i, int j, TF v) { t1[i * NTP + j] = bv[(b0 + i) * NTP + j] - v; }, NTP);
-            __syncthreads();
-            mfma_gemm<false, TF>(nb, nb, I.tmp + f.L1inv + (int64_t)bb * NB * NB, NB, t1, nt,
-                             [&](int i, int j, TF v) { zl[(b0 + i) * NTP + j] = v; }, NTP);
-            __syncthreads();
-        }
-        unstage(I.fac + f.Gz + (int64_t)j0 * nk, nk, zl, 0, nk, nt);
-        unstage(Grc, R, bv, nk, mr, nt);  // (Q_ql' b)[nk:m]
-    } else {
-        unstage(Grc, R, bv, 0, m, nt);  // nothing eliminated: reduced b = b
-    }
-    // u part: W_1' u_1 + W_2' u_2 (ulvfactor.jl:89); a leaf has none
-    if (kv > 0) {
-        TF* Gu = Grc + mr;
-        if (nd.is_leaf) {
-            for (int e = threadIdx.x; e < kv * nt; e += blockDim.x) Gu[(e % kv) + (int64_t)(e / kv) * R] = TF(0);
-        } else {
-            const DevNode dl = I.nodes[nd.left], dr = I.nodes[nd.right];
-            gemm<true>(kv, nt, kvl, I.blob + dl.W, kvl, us, [&](int i, int j, TF v) { t2[i * NTP + j] = v; });
-            __syncthreads();
-            gemm<true>(kv, nt, kvr, I.blob + dr.W, kvr, us + kvl * NTP,
-                       [&](int i, int j, TF v) { Gu[i + (int64_t)j * R] = t2[i * NTP + j] + v; });
-        }
-    }
-}
-
-// Qt = Q_lq' explicitly (ulvfactor.jl:102): column c is H(1)...H(nk) e_c, applied
-// as blocks of NB reflectors z - Y_b T_b Y_b' z, the last block first.
-// LDS: z n x NTP | t1, t2 NB x NTP
-template <typename TF>
-__global__ __launch_bounds__(SWEEP_THREADS) void k_ulv_qform(const FInst<TF>* __restrict__ insts,
-                                                            const WorkItem* __restrict__ work) {
-    const WorkItem wi = work[blockIdx.x];
-    const FInst<TF>& I = insts[wi.inst];
-    const FNode f = I.fn[wi.node];
-    if (f.Qt < 0) return;
-    const int n = f.n;
-    const int j0 = blockIdx.y * RHS_TILE;
-    if (j0 >= n) return;
-    const int nt = min(RHS_TILE, n - j0);
-    const int nk = f.nk;
-    extern __shared__ unsigned char lds_raw[];
-    TF* z = reinterpret_cast<TF*>(lds_raw);
-    TF* t1 = z + n * NTP;
-    TF* t2 = t1 + NB * NTP;
-    for (int e = threadIdx.x; e < n * NTP; e += blockDim.x) {
-        const int r = e / NTP, j = e % NTP;
-        z[e] = (j < nt && r == j0 + j) ? TF(1) : TF(0);
-    }
-    __syncthreads();
-    for (int bb = f.nblk - 1; bb >= 0; --bb) {
-        const int b0 = bb * NB, nb = min(NB, nk - b0);
-        const TF* Yb = I.tmp + f.Ylq + (int64_t)b0 * n + b0;  // rows b0.., columns b0..b0+nb
-        mfma_gemm<true, TF>(nb, n - b0, Yb, n, z + b0 * NTP, nt, [&](int i, int j, TF v) { t1[i * NTP + j] = v; }, NTP);
-        __syncthreads();
-        mfma_gemm<false, TF>(nb, nb, I.tmp + f.Tlq + (int64_t)bb * NB * NB, NB, t1, nt,
-                         [&](int i, int j, TF v) { t2[i * NTP + j] = v; }, NTP);
-        __syncthreads();
-        mfma_gemm<false, TF>(n - b0, nb, Yb, n, t2, nt, [&](int i, int j, TF v) { z[(b0 + i) * NTP + j] -= v; }, NTP);
-        __syncthreads();
-    }
-    unstage(I.fac + f.Qt + (int64_t)j0 * n, n, z, 0, n, nt);
-}
-
 // acc += op(A)(i0 + li, k0 + .) x over the 16 rows of one accumulator-layout tile x (rows
 // k0 .. k0 + 15 of a 16-column block), masked to M x K; A column-major, op = ' when TA.
 // The accumulator layout is the B operand's, so a product's result feeds the next one from
@@ -1553,17 +1406,21 @@ __device__ __forceinline__ typename Mfma<TF>::v4 tile_mac(const TF* __restrict__
     return acc;
 }
 
-// k_ulv_gform and k_ulv_qform for nodes of at most 16 NTILE rows: a wave forms 16 columns of
-// the operator by itself, the column's rows in registers (accumulator layout), every product
-// one MFMA chain with the factor block streamed from memory, no LDS and no barrier.  Unit
-// input columns need no product for the children's merge, the u part and (leaves) Y' b: they
-// are columns of P12 / P21, rows of W and rows of Y.  Bound by the MFMA chain of one wave
-// (about 360 MFMAs, 64 cycles each, for a 128-row leaf).  The LDS kernels run one or two of a
-// workgroup's four waves on the 16-row blocks, with two barriers a block.
-// n = 65536, leaf 128 (1022 nodes): Gz and Gr 370 -> 233 us, Qt 163 -> 143; 32 Cauchy matrices
-// of leaf 64: 961 -> 349 and 187 -> 151 us.
+// k_ulv_gform runs the reduction's steps on columns of the identity (nodes of at most
+// 16 NTILE rows):
+//   Gz (nk x Kx):   column c = zloc for x = e_c
+//   Gr (R x (Kx + nk)), R = mr + kv: column c < Kx = [(Q_ql' b)[nk:m]; W_1'u_1 + W_2'u_2]
+//                   for x = e_c (the reduced b and u before their zloc terms); the last
+//                   nk columns are [-L2a; V_top'], so [reduced b; u] = Gr [x; zloc].
+// A wave forms 16 columns by itself, their rows in registers (accumulator layout), every
+// product one MFMA chain with the factor block streamed from memory, no LDS and no barrier.
+// Unit input columns need no product for the children's merge, the u part and (leaves) Y' b:
+// they are columns of P12 / P21, rows of W and rows of Y.  Bound by the MFMA chain of one wave
+// (about 230 MFMAs, 64 cycles each, for a 128-row leaf of rank 35).  With the columns in LDS
+// and two barriers a 16-row block, one or two of a workgroup's four waves had work in a step.
+// n = 65536, leaf 128 (1022 nodes): 370 -> 233 us; 32 Cauchy matrices of leaf 64: 961 -> 349.
 template <typename TF, int NTILE>
-__global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_gform_w(const FInst<TF>* __restrict__ insts,
+__global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_gform(const FInst<TF>* __restrict__ insts,
                                                                          const WorkItem* __restrict__ work) {
     using MF = Mfma<TF>;
     using V4 = typename MF::v4;
@@ -1692,10 +1549,12 @@ __global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_gform_w(const F
     }
 }
 
-// Qt as k_ulv_qform forms it, 16 columns a wave (see k_ulv_gform_w).  A block of reflectors
-// below a column's unit row leaves it alone, so the wave starts at its own tile's block.
+// Qt = Q_lq' explicitly (ulvfactor.jl:102): column c is H(1)...H(nk) e_c, applied as blocks of
+// NB reflectors z - Y_b T_b Y_b' z, the last block first; 16 columns a wave as above.  A block
+// below a column's unit row leaves it alone, so the wave starts at its own tile's block
+// (163 -> 143 us and 187 -> 151 us on the matrices above).
 template <typename TF, int NTILE>
-__global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_qform_w(const FInst<TF>* __restrict__ insts,
+__global__ __launch_bounds__(256, NTILE <= 4 ? 4 : 2) void k_ulv_qform(const FInst<TF>* __restrict__ insts,
                                                                          const WorkItem* __restrict__ work) {
     using MF = Mfma<TF>;
     using V4 = typename MF::v4;
@@ -2159,16 +2018,13 @@ __device__ __forceinline__ void lds_gemm(int M, int K, const TF* As, const TF* x
 // (lda) in LDS (AL) or in memory, xs row-major in LDS (pitch xp).  A strip covers all
 // (one or two) 16-column blocks, so every A element is read by one wave and feeds one
 // MFMA per column block; with one block the k-steps alternate between acc0 and acc1.
-// TA (A in memory only): the strip's rows are columns of A, i.e. the product is A' xs with
-// A (K x M) column-major (lda).
 // A in memory is loaded straight into registers U k-steps ahead of the MFMAs; the loads
 // are unconditional (columns past K are clamped in bounds and k past K is zeroed at the
 // MFMA), so no wait is forced before a value is used.  Rows past M read row M - 1 and
 // are never stored.
-template <bool AL, bool two, typename TF, bool TA = false>
+template <bool AL, bool two, typename TF>
 __device__ __forceinline__ void strip_acc(int M, int K, const TF* __restrict__ A, int64_t lda, const TF* xs, int xp,
                                           int rb, typename Mfma<TF>::v4& acc0, typename Mfma<TF>::v4& acc1) {
-    static_assert(!(AL && TA), "a transposed A is read from memory only");
     if (K <= 0) return;
     const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
     const int i = rb * 16 + lr;
@@ -2226,11 +2082,11 @@ __device__ __forceinline__ void strip_acc(int M, int K, const TF* __restrict__ A
     // VGPRs per step.  Every access is inside A: the lane's column is clamped to K - 1
     // (full steps never need it) and steps at or past Sf are loaded by the edge code.
     const int kl = lk < K ? lk : K - 1;
-    // element (row i, column k) of the strip's operator: A[i + k lda], or A[k + i lda] (TA)
-    auto at = [&](int i, int k) { return TA ? i * (int)lda + k : i + k * (int)lda; };
+    // element (row i, column k) of the strip's operator
+    auto at = [&](int i, int k) { return i + k * (int)lda; };
     const int voff = at(ic, kl) * (int)sizeof(TF);
-    const int step = 4 * (TA ? 1 : (int)lda) * (int)sizeof(TF);
-    const auto rsrc = buf_rsrc(A, (int)((TA ? lda * (M - 1) + K : lda * (K - 1) + M) * (int64_t)sizeof(TF)));
+    const int step = 4 * (int)lda * (int)sizeof(TF);
+    const auto rsrc = buf_rsrc(A, (int)((lda * (K - 1) + M) * (int64_t)sizeof(TF)));
     auto ld = [&](int st) { return buf_load<TF>(rsrc, voff, (st < Sf ? st : (Sf > 0 ? Sf - 1 : 0)) * step); };
     auto ld_edge = [&](int st) {
         const int kk = 4 * st + lk;
@@ -2323,25 +2179,6 @@ __device__ __forceinline__ void glb_gemm(int M, int K, const TF* __restrict__ A,
                                          Store store, int xp = XS) {
     if (ncols > 16) glb_gemm_cb<true>(M, K, A, lda, xs, ncols, store, xp);
     else glb_gemm_cb<false>(M, K, A, lda, xs, ncols, store, xp);
-}
-
-// out = op(A) xs on MFMA (M x ncols, ncols <= 32; K terms): op(A) = A (M x K, lda), or A'
-// with A (K x M, lda) when TA; xs row-major in LDS (pitch xp).  No barrier inside.
-template <bool TA, typename TF, typename Store>
-__device__ __forceinline__ void mfma_gemm(int M, int K, const TF* __restrict__ A, int64_t lda, const TF* xs, int ncols,
-                                          Store store, int xp) {
-    using V4 = typename Mfma<TF>::v4;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    for (int rb = wave; rb < (M + 15) / 16; rb += nw) {
-        V4 a0 = V4{TF(0), TF(0), TF(0), TF(0)}, a1 = a0;
-        if (ncols > 16) {
-            strip_acc<false, true, TF, TA>(M, K, A, lda, xs, xp, rb, a0, a1);
-            strip_put<true, TF>(M, ncols, rb, lane, a0, a1, store);
-        } else {
-            strip_acc<false, false, TF, TA>(M, K, A, lda, xs, xp, rb, a0, a1);
-            strip_put<false, TF>(M, ncols, rb, lane, a0, a1, store);
-        }
-    }
 }
 
 // The two products of a node's up-sweep step with the input x in xs rows [0, Kx):
@@ -3030,39 +2867,19 @@ hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwor
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_ulv_gform(const FInst<T>* insts, const WorkItem* work, int nwork, int max_kx, size_t lds,
-                            hipStream_t st) {
-    if (nwork <= 0 || max_kx <= 0) return hipSuccess;
-    const void* fn = reinterpret_cast<const void*>(&k_ulv_gform<T>);
-    hipError_t e = set_lds_attr<T>(fn, lds);
-    if (e != hipSuccess) return e;
-    klaunch((k_ulv_gform<T>), dim3(nwork, rhs_tiles(max_kx)), dim3(SWEEP_THREADS), lds, st, insts, work);
-    return hipGetLastError();
-}
-template <typename T>
-hipError_t launch_ulv_qform(const FInst<T>* insts, const WorkItem* work, int nwork, int max_n, size_t lds,
-                            hipStream_t st) {
-    if (nwork <= 0 || max_n <= 0) return hipSuccess;
-    const void* fn = reinterpret_cast<const void*>(&k_ulv_qform<T>);
-    hipError_t e = set_lds_attr<T>(fn, lds);
-    if (e != hipSuccess) return e;
-    klaunch((k_ulv_qform<T>), dim3(nwork, rhs_tiles(max_n)), dim3(SWEEP_THREADS), lds, st, insts, work);
-    return hipGetLastError();
-}
-template <typename T>
-hipError_t launch_ulv_forms_w(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, int max_kx, int max_n,
+hipError_t launch_ulv_forms(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, int max_kx, int max_n,
                               hipStream_t st) {
     if (nwork <= 0) return hipSuccess;
-    if (max_m > FORM_W_ROWS || max_n > FORM_W_ROWS) return hipErrorInvalidValue;
+    if (max_m > 128 || max_n > 128) return hipErrorInvalidValue;
     const bool small = max_m <= 64;
     const int gy = (max_kx + 63) / 64, qy = (max_n + 63) / 64;
     if (gy > 0) {
-        if (small) klaunch((k_ulv_gform_w<T, 4>), dim3(nwork, gy), dim3(256), 0, st, insts, work);
-        else klaunch((k_ulv_gform_w<T, 8>), dim3(nwork, gy), dim3(256), 0, st, insts, work);
+        if (small) klaunch((k_ulv_gform<T, 4>), dim3(nwork, gy), dim3(256), 0, st, insts, work);
+        else klaunch((k_ulv_gform<T, 8>), dim3(nwork, gy), dim3(256), 0, st, insts, work);
     }
     if (qy > 0) {
-        if (small) klaunch((k_ulv_qform_w<T, 4>), dim3(nwork, qy), dim3(256), 0, st, insts, work);
-        else klaunch((k_ulv_qform_w<T, 8>), dim3(nwork, qy), dim3(256), 0, st, insts, work);
+        if (small) klaunch((k_ulv_qform<T, 4>), dim3(nwork, qy), dim3(256), 0, st, insts, work);
+        else klaunch((k_ulv_qform<T, 8>), dim3(nwork, qy), dim3(256), 0, st, insts, work);
     }
     return hipGetLastError();
 }
@@ -3843,9 +3660,7 @@ template hipError_t launch_ulv_wy<float>(const FInst<float>*, const WorkItem*, i
 template hipError_t launch_ulv_root<double>(const FInst<double>*, const WorkItem*, int, int, hipStream_t);
 template hipError_t launch_ulv_root<float>(const FInst<float>*, const WorkItem*, int, int, hipStream_t);
 #define HSS_INST_SOLVE(T)                                                                                      \
-    template hipError_t launch_ulv_gform<T>(const FInst<T>*, const WorkItem*, int, int, size_t, hipStream_t);       \
-    template hipError_t launch_ulv_qform<T>(const FInst<T>*, const WorkItem*, int, int, size_t, hipStream_t);       \
-    template hipError_t launch_ulv_forms_w<T>(const FInst<T>*, const WorkItem*, int, int, int, int, hipStream_t);   \
+    template hipError_t launch_ulv_forms<T>(const FInst<T>*, const WorkItem*, int, int, int, int, hipStream_t);   \
     template hipError_t launch_ulv_gup<T>(const SInst<T>*, const SweepRec*, int, int, int, hipStream_t);            \
     template hipError_t launch_ulv_groot<T>(const SInst<T>*, const SweepRec*, int, int, size_t, int, hipStream_t);   \
     template hipError_t launch_ulv_rinv<T>(const FInst<T>*, const WorkItem*, int, int, size_t, hipStream_t);       \

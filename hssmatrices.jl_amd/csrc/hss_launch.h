@@ -48,17 +48,11 @@ hipError_t launch_ulv_wy(const FInst<T>* insts, const WorkItem* work, int nwork,
 template <typename T>
 hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, hipStream_t st);
 // solve operators, once per factorization (every non-root node in one launch)
-// Gz, Gr and Qt of nodes with at most FORM_W_ROWS rows (k_ulv_gform_w, k_ulv_qform_w)
-constexpr int FORM_W_ROWS = 128;
+// Gz, Gr and Qt of nodes with at most 128 rows (k_ulv_gform, k_ulv_qform); the factor kernels
+// take no larger ones: m S <= FACT_THREADS, and S = 8 from n = 129 on
 template <typename T>
-hipError_t launch_ulv_forms_w(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, int max_kx, int max_n,
+hipError_t launch_ulv_forms(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, int max_kx, int max_n,
                               hipStream_t st);
-template <typename T>
-hipError_t launch_ulv_gform(const FInst<T>* insts, const WorkItem* work, int nwork, int max_kx, size_t lds,
-                            hipStream_t st);
-template <typename T>
-hipError_t launch_ulv_qform(const FInst<T>* insts, const WorkItem* work, int nwork, int max_n, size_t lds,
-                            hipStream_t st);
 // solve sweeps: max_nk = largest nk (up), max_m = largest n (down) of the level's nodes
 template <typename T>
 hipError_t launch_ulv_gup(const SInst<T>* insts, const SweepRec* work, int nwork, int max_nk, int max_nrhs,

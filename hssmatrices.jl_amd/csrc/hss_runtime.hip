@@ -406,7 +406,6 @@ struct hss_fact_s {
     size_t lds_groot_res = 0;          // the same with the root's factor staged in LDS
     size_t lds_groot2 = 0;             // the inverse-and-refine root kernel (0: not available)
     size_t lds_groot2s = 0;            // the same with D and Mb staged too
-    size_t lds_gform = 0, lds_qform = 0;
     void* d_wy = nullptr;  // y blocks, then the z blocks at wy + yrows * nrhs
     size_t ws_cap = 0;     // nrhs capacity
     SlotCache sinst;
@@ -1927,8 +1926,9 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
     }
     F->yrows = yrows;
     F->zrows = zrows;
-    // LDS (rows of NTP = RHS_TILE columns) and widths of the operator-forming kernels
-    size_t gform = 0, qform = 0, groot = 0;
+    // LDS (rows of NTP = RHS_TILE columns) of the root kernels, and the largest node (rows and
+    // ranks) that the library takes
+    size_t most = 0, groot = 0;
     for (int i = 0; i < nn; ++i) {
         const FNode& f = F->hfn[i];
         const DevNode& d = M->hn[i];
@@ -1937,13 +1937,10 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
             groot = (size_t)f.m + kvc + NB;
         } else {
             const size_t tr = (size_t)std::max(std::max(f.k, NB), d.kv);
-            gform = std::max(gform, (size_t)f.m + std::max(f.nk, 1) + kvc + 2 * tr);
-            qform = std::max(qform, (size_t)f.n + 2 * NB);
+            most = std::max(most, (size_t)f.m + std::max(f.nk, 1) + kvc + 2 * tr);
         }
     }
     const size_t tv = sizeof(TF) * RHS_TILE;
-    F->lds_gform = gform * tv;
-    F->lds_qform = qform * tv;
     F->lds_groot = groot * tv;
     F->lds_groot_res = groot * tv + sizeof(TF) * (size_t)((fr.rlen + 15) & ~int64_t(15));
     if (fr.Dinv >= 0) {
@@ -1951,7 +1948,7 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
         F->lds_groot2 = sizeof(TF) * (size_t)(((int64_t)fr.m * fr.m + 15) / 16 * 16 + io);
         F->lds_groot2s = sizeof(TF) * (size_t)((2 * (int64_t)fr.m * fr.m + (int64_t)fr.m * fr.Kx + 15) / 16 * 16 + io);
     }
-    if (F->lds_gform > 160 * 1024 || F->lds_groot > 160 * 1024)
+    if (most * tv > 160 * 1024 || F->lds_groot > 160 * 1024)
         return fail(HSS_ERR_UNSUPPORTED, "a node exceeds the LDS of the solve-operator kernels");
     return HSS_OK;
 }
@@ -2036,11 +2033,9 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
         s = alloc_resident<TF>(F);
         if (s != HSS_OK) { cleanup(); return s; }
     }
-    size_t lds_gform = 0, lds_qform = 0, lds_rinv = 0;
+    size_t lds_rinv = 0;
     int max_rcols = 0, max_rm = 0;
     for (auto* F : out) {
-        lds_gform = std::max(lds_gform, F->lds_gform);
-        lds_qform = std::max(lds_qform, F->lds_qform);
         const FNode& r = F->hfn[0];
         max_rm = std::max(max_rm, r.m);
         if (r.Dinv >= 0) {
@@ -2083,19 +2078,18 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
                lev_lds_mf[h] <= 160 * 1024;
     };
     const int nonroot = (int)work.size();  // every non-root node of every matrix
-    // The operator-forming kernels by size: a wave per 16 columns with the rows in registers
-    // up to 64 and up to FORM_W_ROWS rows (a 64-row node in the 128-row build would run twice
-    // the tiles), the LDS kernels beyond.
+    // The operator-forming kernels by size: nodes of up to 64 rows run the build that holds
+    // four tiles (in the eight-tile one they would run twice the MFMAs, at half the waves).
     struct FormClass {
         Range r;
         int m = 0, kx = 0, nq = 0;
-    } form[3];
-    for (int c = 0; c < 3; ++c) {
+    } form[2];
+    for (int c = 0; c < 2; ++c) {
         form[c].r.off = (int)work.size();
         for (int e = 0; e < nonroot; ++e) {
             const WorkItem w = work[e];
             const FNode& f = out[w.inst]->hfn[w.node];
-            if ((f.m <= 64 ? 0 : f.m <= FORM_W_ROWS ? 1 : 2) != c) continue;
+            if ((f.m > 64) != (c == 1)) continue;
             work.push_back(w);
             form[c].m = std::max(form[c].m, f.m);
             form[c].kx = std::max(form[c].kx, f.Kx + f.nk);
@@ -2170,13 +2164,8 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
         // solve operators G and Qt of every non-root node (one launch each)
         for (int c = 0; c < 2; ++c) {
             ProfScope ps("k_ulv_forms", c, form[c].r.count, st);
-            HIP_TRY((launch_ulv_forms_w<TF>(d_inst, d_work + form[c].r.off, form[c].r.count, form[c].m, form[c].kx,
+            HIP_TRY((launch_ulv_forms<TF>(d_inst, d_work + form[c].r.off, form[c].r.count, form[c].m, form[c].kx,
                                             form[c].nq, st)));
-        }
-        if (form[2].r.count > 0) {
-            ProfScope ps("k_ulv_gform", 0, form[2].r.count, st);
-            HIP_TRY((launch_ulv_gform<TF>(d_inst, d_work + form[2].r.off, form[2].r.count, form[2].kx, lds_gform, st)));
-            HIP_TRY((launch_ulv_qform<TF>(d_inst, d_work + form[2].r.off, form[2].r.count, form[2].nq, lds_qform, st)));
         }
         HIP_TRY(hipEventRecord(ctx->ev1, st));
         HIP_TRY(hipMemcpyAsync(info.data(), d_info, sizeof(int32_t) * cnt, hipMemcpyDeviceToHost, st));
