@@ -1313,6 +1313,9 @@ __global__ __launch_bounds__(ROOT_THREADS) void k_ulv_root(const FInst<T>* __res
         const T pv = A[p + i * lda];
         if (tid == 0) piv[i] = p;
         if (pv == T(0) || pv != pv) {  // a zero or NaN pivot: singular (status i + 1)
+            // k_ulv_rinv, already enqueued, exchanges rows by every entry of piv before the
+            // status is looked at: the rest of them stay where they are
+            for (int q = i + 1 + tid; q < m; q += blockDim.x) piv[q] = q;
             info = i + 1;
             break;
         }
