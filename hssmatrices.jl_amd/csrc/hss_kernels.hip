@@ -659,49 +659,50 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
         }
     }
     // ---- phase 2: M = T (Y' D), so that Q_ql' D = D - Y M  (ulvfactor.jl:41) ----
-    // A wave takes 16 columns of D through both products on MFMA: Y' D (four tiles of
-    // reflectors at a time, 64 rows of D in flight, lane lk taking four adjacent rows) into M,
-    // then T times it.  Bound by the MFMA chain (96 for 128 x 128 and rank 35) and one trip to
-    // memory; a dot product a thread with lane shuffles took 14-47 us a node.
+    // A wave takes 16 columns of D through both products on MFMA: Y' D (64 rows of D in
+    // flight, lane lk taking four adjacent rows) into M, then T times it.  Bound by the MFMAs (96
+    // for 128 x 128 and rank 35) and one trip to memory; a dot product a thread with lane
+    // shuffles took 14-47 us a node.  Y' D is added up as partial sums of 16 rows: one
+    // accumulator over all m rows gave 1.1-1.2 times the error of the whole solve (5.9e-15
+    // instead of 5.0e-15 at n = 65536, 2.0e-13 instead of 1.5e-13 on Cauchy matrices) in the
+    // same time.
     {
         using MF = Mfma<T>;
         using V4 = typename MF::v4;
-        const int li = lane & 15, lk = lane >> 4, kt = (k + 15) / 16;
-        auto yt = [&](int c0, int q0) {  // Y' D for one column tile and reflector tiles q0 .. q0 + 3
+        // formed here again: with tid held from the start of the kernel the four-tile build
+        // spills it, and reloading it costs 3 % of a launch
+        const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4, kt = (k + 15) / 16;
+        for (int c0 = 16 * wv; c0 < n; c0 += 16 * nwaves) {
             const int c = c0 + li, cc = min(c, n - 1);
-            V4 acc[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q] = V4{T(0), T(0), T(0), T(0)};
             for (int i0 = 0; i0 < m; i0 += 64) {
                 T d[16];
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const int i = i0 + 16 * (e >> 2) + 4 * lk + (e & 3);
                     const T v = Wsrc(min(i, m - 1), cc);
-                    d[e] = i < m && c < n ? v : T(0);
+                    d[e] = i < m ? v : T(0);
                 }
+#pragma unroll 1
+                for (int q = 0; q < kt; ++q) {
+                    const int jc = min(16 * q + li, k - 1);
+                    V4 s[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if (q0 + q >= kt) continue;
-                    const int j = 16 * (q0 + q) + li, jc = min(j, k - 1);
+                    for (int h = 0; h < 4; ++h) s[h] = V4{T(0), T(0), T(0), T(0)};
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         const int i = i0 + 16 * (e >> 2) + 4 * lk + (e & 3);
-                        const T y = yql(min(i, m - 1), jc);
-                        acc[q] = MF::mac(i < m && j < k ? y : T(0), d[e], acc[q]);
+                        s[e & 3] = MF::mac(yql(min(i, m - 1), jc), d[e], s[e & 3]);
+                    }
+                    const V4 sum = (s[0] + s[1]) + (s[2] + s[3]);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int jo = 16 * q + MF::row(lk, r);
+                        if (jo < k && c < n) Mq[jo * vstride + vpad<CPT>(c)] += sum[r];
                     }
                 }
             }
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int j = 16 * (q0 + q) + MF::row(lk, r);
-                    if (j < k && c < n) Mq[j * vstride + vpad<CPT>(c)] = acc[q][r];
-                }
-        };
-        for (int c0 = 16 * wave; c0 < n; c0 += 16 * nwaves)
-            for (int q0 = 0; q0 < kt; q0 += 4) yt(c0, q0);
+        }
         __syncthreads();  // T
         {
             T* Tg = I.tmp + f.Tql;
@@ -709,7 +710,7 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
         }
         // M <- T M in place, the wave's own columns (T upper triangular: ascending tiles read
         // only rows at and below their own)
-        for (int c0 = 16 * wave; c0 < n; c0 += 16 * nwaves) {
+        for (int c0 = 16 * wv; c0 < n; c0 += 16 * nwaves) {
             const int c = c0 + li;
             const T* mc = Mq + vpad<CPT>(min(c, n - 1));
             for (int q = 0; q < kt; ++q) {
