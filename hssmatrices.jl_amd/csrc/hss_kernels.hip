@@ -694,7 +694,7 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
                         const int i = i0 + 16 * (e >> 2) + 4 * lk + (e & 3);
                         s[e & 3] = MF::mac(yql(min(i, m - 1), jc), d[e], s[e & 3]);
                     }
-                    const V4 sum = (s[0] + s[1]) + (s[2] + s[3]);
+                    const V4 sum = ((s[0] + s[1]) + s[2]) + s[3];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int jo = 16 * q + MF::row(lk, r);

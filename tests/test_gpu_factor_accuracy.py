@@ -4,8 +4,8 @@ all of c 11' out of the rows that are eliminated, so an error of p eps in the su
 about p cond(A) eps in the solution.  With t = 1 the additions are exact, which gives the error of
 everything else (the reflector's scale and tau, the update with Y).  t = 1 + f 2^-46 makes each
 addition to a partial sum in [64 t, 128 t) round the same way by up to half a unit: one running sum
-over the 128 rows adds up to 14 eps.  Partial sums of 16 rows, added pairwise, lose at most 2.7 eps
-in the sums and 1.5 in adding them."""
+over the 128 rows adds up to 14 eps.  Partial sums of 16 rows lose at most 2.7 eps in the sums
+and 1.5 in adding them up."""
 import numpy as np
 import pytest
 
