@@ -2502,6 +2502,9 @@ static hss_status ensure_refine(hss_fact_s* F, int nrhs) {
     return HSS_OK;
 }
 
+// The larger of two relative residuals; a NaN stays the worst (as in k_refine_check).
+static double worse(double a, double b) { return b > a || b != b ? b : a; }
+
 // R = B - R (R holds A X on entry); *out = max_j ||r_j|| / ||b_j||
 static hss_status residual_norm(hss_fact_s* F, int nrhs, const double* dB, int64_t ldb, double* dR, int64_t ldr,
                                 hipStream_t st, double* out) {
@@ -2517,7 +2520,7 @@ static hss_status residual_norm(hss_fact_s* F, int nrhs, const double* dB, int64
     for (int j = 0; j < nrhs; ++j) {
         const double nb = std::sqrt(h[2 * j]), nr = std::sqrt(h[2 * j + 1]);
         const double rel = nb > 0 ? nr / nb : nr;
-        worst = std::max(worst, rel);
+        worst = worse(worst, rel);
     }
     *out = worst;
     return HSS_OK;
@@ -2711,7 +2714,7 @@ static hss_status solve_dev_impl(hss_fact_s* F, int nrhs, const double* dB, int6
             g_last_ms = ms;
             if (rep) rep->seconds = ms * 1e-3;
         }
-        if (rel > o.tol) {
+        if (rel > o.tol || rel != rel) {
             char buf[160];
             std::snprintf(buf, sizeof buf, "refinement stopped at relative residual %.3e > tol %.3e after %d steps",
                           rel, o.tol, it);
@@ -3371,7 +3374,7 @@ extern "C" hss_status hss_plan_execute(hss_plan_t P, const hss_refine_opts* opts
     HIP_TRY(hipMemcpy(hrel.data(), P->d_rel, sizeof(double) * P->cnt, hipMemcpyDeviceToHost));
     double worst = 0.0;
     for (int i = 0; i < P->cnt; ++i)
-        if (P->reqs[i].nrhs > 0) worst = hrel[i] > worst || hrel[i] != hrel[i] ? hrel[i] : worst;
+        if (P->reqs[i].nrhs > 0) worst = worse(worst, hrel[i]);
     // the device tables retired requests on their own: upload the full activity again
     P->uploaded_active.assign(P->cnt, 2);
     // restore all requests as active for the next execution
@@ -3727,7 +3730,7 @@ static hss_status server_round(hss_server_s* S) {
         double rel = 0.0;
         for (int j = 0; j < q->nrhs; ++j) {
             const double b2 = norms[2 * ((size_t)i * maxnrhs + j)], r2 = norms[2 * ((size_t)i * maxnrhs + j) + 1];
-            rel = std::max(rel, b2 > 0 ? std::sqrt(r2 / b2) : std::sqrt(r2));
+            rel = worse(rel, b2 > 0 ? std::sqrt(r2 / b2) : std::sqrt(r2));
         }
         q->rel = rel;
         const bool conv = rel <= S->opts.tol || S->opts.mode == 0;
