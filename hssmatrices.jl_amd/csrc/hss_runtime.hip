@@ -2130,12 +2130,14 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
         I.ipiv = out[b]->d_piv;
         I.status = d_info + b;
     }
+    // copied from and to asynchronously, so both outlive run(): the pool waits for the stream below,
+    // also where a launch failed
+    std::vector<char> tab(inst_bytes + sizeof(WorkItem) * work.size());
+    std::memcpy(tab.data(), hinst.data(), sizeof(FInst<TF>) * cnt);
+    std::memcpy(tab.data() + inst_bytes, work.data(), sizeof(WorkItem) * work.size());
     std::vector<int32_t> info(cnt, 0);
     hss_status rs = HSS_OK;
     auto run = [&]() -> hss_status {
-        std::vector<char> tab(inst_bytes + sizeof(WorkItem) * work.size());
-        std::memcpy(tab.data(), hinst.data(), sizeof(FInst<TF>) * cnt);
-        std::memcpy(tab.data() + inst_bytes, work.data(), sizeof(WorkItem) * work.size());
         HIP_TRY(hipMemcpyAsync(d_scratch, tab.data(), tab.size(), hipMemcpyHostToDevice, st));
         HIP_TRY(hipEventRecord(ctx->ev0, st));
         for (int h = 0; h < maxh; ++h) {
