@@ -463,7 +463,7 @@ extern "C" hss_status hss_randcompress_dev(hss_ctx_t ctx, const double* dA, int6
         }
         const int64_t blob_len = pos;
         double* blob = nullptr;
-        CTRY(hipMalloc(reinterpret_cast<void**>(&blob), sizeof(double) * (size_t)std::max<int64_t>(blob_len, 1)));
+        CTRY(dev_malloc(reinterpret_cast<void**>(&blob), sizeof(double) * (size_t)std::max<int64_t>(blob_len, 1)));
         {
             TaskList gt;
             for (int i = 0; i < nn; ++i) {

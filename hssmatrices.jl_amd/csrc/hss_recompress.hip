@@ -490,7 +490,7 @@ extern "C" hss_status hss_mat_recompress(hss_mat_t mat, double atol, double rtol
     }
     const int64_t blob_len = pos;
     double* blob = nullptr;
-    CTRY(hipMalloc(reinterpret_cast<void**>(&blob), sizeof(double) * (size_t)std::max<int64_t>(blob_len, 1)));
+    CTRY(dev_malloc(reinterpret_cast<void**>(&blob), sizeof(double) * (size_t)std::max<int64_t>(blob_len, 1)));
     {
         TaskList g;
         for (int i = 0; i < nn; ++i) {

@@ -28,6 +28,8 @@
 #include "hss_host.h"
 #include "hss_internal.h"
 #include "hss_launch.h"
+#include "hss_pool.h"
+#include "hss_tasks.h"
 
 using namespace hss;
 
@@ -123,11 +125,36 @@ struct ProfScope {
     }
 };
 
+// Device memory for BlockPool; `error` is why the thread's last allocation failed.
+struct HipMem {
+    static thread_local hipError_t error;
+    static void* alloc(size_t bytes) {
+        void* p = nullptr;
+        error = hipMalloc(&p, bytes);
+        if (error == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    static void release(void* p) { (void)hipFree(p); }
+};
+thread_local hipError_t HipMem::error = hipSuccess;
+namespace hss {
+// hipMalloc on the current device; where it fails, the pools of the device's contexts free what they
+// hold and it is tried again
+hipError_t dev_malloc(void** p, size_t bytes) {
+    int device = 0;
+    *p = nullptr;
+    const hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    *p = BlockPool<HipMem>::allocate(device, bytes);
+    return *p ? hipSuccess : HipMem::error;
+}
+}  // namespace hss
+
 template <typename T>
 static hipError_t dalloc(T** p, size_t count) {
-    *p = nullptr;
     if (count == 0) count = 1;
-    return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
+    return dev_malloc(reinterpret_cast<void**>(p), count * sizeof(T));
 }
 
 // ---------------------------------------------------------------------------
@@ -163,7 +190,7 @@ struct SlotCache {
     hipError_t get(const void* v, size_t bytes, hipStream_t st, const void** out) {
         if (!d) {
             rec = bytes;
-            hipError_t e = hipMalloc(reinterpret_cast<void**>(&d), rec * SLOTS);
+            hipError_t e = dev_malloc(reinterpret_cast<void**>(&d), rec * SLOTS);
             if (e != hipSuccess) return e;
             h.assign(rec * SLOTS, 0);
         }
@@ -275,71 +302,27 @@ static hss_status plan_create_impl(int32_t count, hss_fact_s* const* facts, cons
                                    const double* const* dB, const int64_t* ldb, double* const* dX, const int64_t* ldx,
                                    int32_t with_refinement, bool hold, hss_plan_t* out);
 
-// Device memory of factors and plans, which come and go with every `\`: blocks given back are
-// kept for the next request of about their size (at most twice it; sizes are rounded up to an
-// eighth of their power of two, so that matrices with slightly other ranks share them), up to
-// kHeldMax bytes and kHeldBlocks blocks in all, and freed with the context or when an allocation fails.  A block
-// is given back only once the context's stream is idle, as hipFree would have waited.  hipMalloc
-// and hipFree cost tens to hundreds of microseconds each (mapping and unmapping).
+// A context's pool (hss_pool.h): put() waits until the context's stream is idle, as hipFree
+// would have waited.
 class DevPool {
 public:
+    void attach(int dev) { pool.attach(device = dev); }
     template <typename T>
-    hipError_t get(T** p, size_t bytes) {
-        *p = nullptr;
-        size_t step = 4096;
-        while (16 * step <= bytes) step *= 2;
-        bytes = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
-        std::lock_guard<std::mutex> lk(mu);
-        auto it = held.lower_bound(bytes);
-        if (it != held.end() && it->first <= 2 * bytes) {
-            *p = static_cast<T*>(it->second);
-            held_bytes -= it->first;
-            used[it->second] = it->first;
-            held.erase(it);
-            return hipSuccess;
-        }
-        void* d = nullptr;
-        hipError_t e = hipMalloc(&d, bytes);
-        if (e != hipSuccess && !held.empty()) {
-            (void)hipGetLastError();
-            trim_locked();
-            e = hipMalloc(&d, bytes);
-        }
-        if (e != hipSuccess) return e;
-        used[d] = bytes;
-        *p = static_cast<T*>(d);
-        return hipSuccess;
+    hipError_t get(T** p, size_t bytes, bool exact = false, size_t* got = nullptr) {
+        HipMem::error = hipErrorOutOfMemory;  // of the host, where the device had the block
+        *p = static_cast<T*>(pool.get(device, bytes, exact, got));
+        return *p ? hipSuccess : (HipMem::error != hipSuccess ? HipMem::error : hipErrorOutOfMemory);
     }
     void put(void* p, hipStream_t st) {
         if (!p) return;
         (void)hipStreamSynchronize(st);
-        std::lock_guard<std::mutex> lk(mu);
-        const auto it = used.find(p);
-        const size_t bytes = it->second;
-        used.erase(it);
-        if (held_bytes + bytes > kHeldMax || held.size() >= kHeldBlocks) {
-            (void)hipFree(p);
-            return;
-        }
-        held.emplace(bytes, p);
-        held_bytes += bytes;
+        pool.put(p);
     }
-    void trim() {
-        std::lock_guard<std::mutex> lk(mu);
-        trim_locked();
-    }
+    bool trim() { return pool.trim(); }
 
 private:
-    static constexpr size_t kHeldMax = size_t(2) << 30, kHeldBlocks = 512;
-    void trim_locked() {
-        for (auto& h : held) (void)hipFree(h.second);
-        held.clear();
-        held_bytes = 0;
-    }
-    std::mutex mu;
-    std::multimap<size_t, void*> held;
-    std::map<void*, size_t> used;
-    size_t held_bytes = 0;
+    int device = 0;
+    BlockPool<HipMem> pool;
 };
 
 // Handles hold references on what they use (a matrix on its context, a factor on
@@ -469,6 +452,7 @@ extern "C" hss_status hss_ctx_create(int device, hss_ctx_t* out) {
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIP_TRY(hipEventCreate(&c->ev0));
     HIP_TRY(hipEventCreate(&c->ev1));
+    c->pool.attach(device);
     *out = c;
     return HSS_OK;
 }
@@ -477,7 +461,6 @@ static void ctx_release(hss_ctx_s* c) {
     if (!c || --c->refs > 0) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    c->pool.trim();
     (void)hipEventDestroy(c->ev0);
     (void)hipEventDestroy(c->ev1);
     (void)hipStreamDestroy(c->stream);
@@ -485,6 +468,13 @@ static void ctx_release(hss_ctx_s* c) {
 }
 extern "C" hss_status hss_ctx_destroy(hss_ctx_t c) {
     ctx_release(c);
+    return HSS_OK;
+}
+
+extern "C" hss_status hss_ctx_trim(hss_ctx_t c) {
+    if (!c) return fail(HSS_ERR_ARG, "null context");
+    HIP_TRY(hipSetDevice(c->device));
+    c->pool.trim();
     return HSS_OK;
 }
 
@@ -1966,17 +1956,22 @@ static void free_fact(hss_fact_s* F) {
 static void build_schedule(const std::vector<hss_fact_s*>& facts, Schedule& S);
 static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
+// what a pool's block holds beyond the request, past the last page
+static int64_t pool_extra(size_t asked, size_t got) { return (int64_t)(got - BlockPool<HipMem>::rounded(asked, true)); }
+
 // The factor's own device memory, one allocation: the resident operators (16 elements of
 // slack for whole-vector loads), the node table, the single-request solve schedule (so that
-// solves, the allocation-free one included, find it ready) and the root's pivots.
+// solves, the allocation-free one included, find it ready) and the root's pivots.  `exact`: a
+// block of that size and no larger (a server's factors, which stay).
 template <typename TF>
-static hss_status alloc_resident(hss_fact_s* F) {
+static hss_status alloc_resident(hss_fact_s* F, bool exact) {
     build_schedule(std::vector<hss_fact_s*>{F}, F->sched);
     const size_t fn_b = sizeof(FNode) * F->hfn.size(), sw_b = sizeof(SweepRec) * F->sched.rec.size();
     const size_t at_fn = align256(sizeof(TF) * ((size_t)F->res_len + 16)), at_sw = align256(at_fn + fn_b),
                  at_piv = align256(at_sw + sw_b), total = at_piv + sizeof(int32_t) * ((size_t)F->hfn[0].m + 1);
     char* d = nullptr;
-    const hipError_t e = F->mat->ctx->pool.get(&d, total);
+    size_t got = 0;
+    const hipError_t e = F->mat->ctx->pool.get(&d, total, exact, &got);
     if (e != hipSuccess) return fail(HSS_ERR_OOM, std::string("factor allocation: ") + hipGetErrorString(e));
     F->d_fac = d;
     F->d_fn = reinterpret_cast<FNode*>(d + at_fn);
@@ -1986,14 +1981,15 @@ static hss_status alloc_resident(hss_fact_s* F) {
     std::memcpy(tab.data(), F->hfn.data(), fn_b);
     std::memcpy(tab.data() + (at_sw - at_fn), F->sched.rec.data(), sw_b);
     HIP_TRY(hipMemcpy(d + at_fn, tab.data(), tab.size(), hipMemcpyHostToDevice));
-    F->dev_bytes = (int64_t)(sizeof(TF) * F->res_len + fn_b + 4 * (F->hfn[0].m + 1));
+    F->dev_bytes = (int64_t)(sizeof(TF) * F->res_len + fn_b + 4 * (F->hfn[0].m + 1)) + pool_extra(total, got);
     return HSS_OK;
 }
 
 // Factor a batch of matrices that share one context: one launch per height
 // across all of them, then one root launch.
 template <typename TF>
-static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec prec, std::vector<hss_fact_s*>& out) {
+static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec prec, std::vector<hss_fact_s*>& out,
+                               bool exact = false) {
     const int cnt = (int)mats.size();
     hss_ctx_s* ctx = mats[0]->ctx;
     hipStream_t st = ctx->stream;
@@ -2030,7 +2026,7 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
         maxh = std::max(maxh, M->max_height);
         tmp_off[b] = tmp_total;
         tmp_total += (F->tmp_len + 15) & ~int64_t(15);
-        s = alloc_resident<TF>(F);
+        s = alloc_resident<TF>(F, exact);
         if (s != HSS_OK) { cleanup(); return s; }
     }
     size_t lds_rinv = 0;
@@ -2925,8 +2921,9 @@ static hss_status plan_tables(hss_plan_s* P) {
             tot = align256(tot + sizeof(double) * (size_t)M->rows * q.nrhs);
         }
     }
-    HIP_TRY(P->ctx->pool.get(&P->arena, std::max<size_t>(tot, 256)));
-    P->dev_bytes = (int64_t)tot;
+    size_t got = 0;
+    HIP_TRY(P->ctx->pool.get(&P->arena, std::max<size_t>(tot, 256), false, &got));
+    P->dev_bytes = (int64_t)tot + pool_extra(std::max<size_t>(tot, 256), got);
     P->sinst_size = sizeof(SInst<TF>);
     for (int t = 0; t < (P->has_ir ? 2 : 1); ++t) {
         std::vector<SInst<TF>> v(cnt);
@@ -3523,7 +3520,7 @@ static hss_status grow(char** p, size_t* cap, size_t need) {
     *cap = 0;
     size_t c = std::max(need, (size_t)1 << 20);
     c = std::max(c, need + need / 2);
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(p), c));
+    HIP_TRY(dev_malloc(reinterpret_cast<void**>(p), c));
     *cap = c;
     return HSS_OK;
 }
@@ -3558,9 +3555,13 @@ extern "C" hss_status hss_server_admit(hss_server_t S, hss_mat_t mat, int32_t* i
     if (S->used + estimate > S->budget)
         return fail(HSS_ERR_BUDGET, "admission refused: " + std::to_string(S->used + estimate) + " bytes > budget " +
                                         std::to_string(S->budget));
-    hss_fact_t F = nullptr;
-    hss_status st = hss_ulv_factor(mat, S->prec, &F);
+    HIP_TRY(hipSetDevice(S->ctx->device));
+    std::vector<hss_fact_s*> f;
+    const std::vector<hss_mat_s*> m{mat};
+    const hss_status st = S->prec == HSS_PREC_FP32 ? factor_batch<float>(m, S->prec, f, true)
+                                                   : factor_batch<double>(m, S->prec, f, true);
     if (st != HSS_OK) return st;
+    hss_fact_t F = f[0];
     const int64_t bytes = F->dev_bytes;
     if (S->used + bytes > S->budget) {
         hss_fact_destroy(F);
@@ -3618,7 +3619,7 @@ static hss_status server_round(hss_server_s* S) {
         hss_mat_s* M = S->facts[q->mid]->mat;
         const size_t bytes = sizeof(double) * 2 * (size_t)M->rows * q->nrhs;
         if (S->used + (int64_t)bytes > S->budget && !S->inflight.empty()) break;  // wait for memory to free up
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&q->r), bytes));
+        HIP_TRY(dev_malloc(reinterpret_cast<void**>(&q->r), bytes));
         q->d = q->r + (size_t)M->rows * q->nrhs;
         q->rbytes = bytes;
         S->used += (int64_t)bytes;

@@ -11,6 +11,9 @@
 
 namespace hss {
 
+// hipMalloc that makes the pools of the device's contexts give back what they hold before it fails
+hipError_t dev_malloc(void** p, size_t bytes);
+
 // device buffers of one compression, freed together after the stream has drained
 struct Buffers {
     hipStream_t st = nullptr;
@@ -22,7 +25,7 @@ struct Buffers {
     template <typename T>
     hipError_t get(T** p, size_t count) {
         void* q = nullptr;
-        hipError_t e = hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T));
+        hipError_t e = dev_malloc(&q, std::max<size_t>(count, 1) * sizeof(T));
         if (e != hipSuccess) return e;
         ptrs.push_back(q);
         *p = reinterpret_cast<T*>(q);

@@ -46,7 +46,7 @@ PREC_FP64, PREC_FP32 = 0, 1
 
 # every symbol include/hss_hip.h declares
 EXPORTS = [
-    "hss_ctx_create", "hss_ctx_destroy", "hss_ctx_stream",
+    "hss_ctx_create", "hss_ctx_destroy", "hss_ctx_trim", "hss_ctx_stream",
     "hss_mat_create", "hss_mat_destroy", "hss_mat_adjoint", "hss_mat_mul", "hss_mat_size", "hss_mat_device_bytes",
     "hss_gen_write", "hss_gen_read", "hss_mat_load", "hss_mat_save", "hss_compress_dev", "hss_randcompress_dev", "hss_mat_recompress", "hss_mat_ldiv", "hss_mat_rdiv", "hss_mat_generators",
     "hss_mat_create_f32", "hss_matmul_f32", "hss_ulvfactsolve_f32", "hss_ulv_solve_f32",
@@ -100,6 +100,7 @@ def load_library(path: pathlib.Path | str | None = None):
     sig = {
         "hss_ctx_create": ([ctypes.c_int, PV], ctypes.c_int),
         "hss_ctx_destroy": ([V], ctypes.c_int),
+        "hss_ctx_trim": ([V], ctypes.c_int),
         "hss_ctx_stream": ([V], V),
         "hss_mat_create": ([V, V, I32, V, I64, PV], ctypes.c_int),
         "hss_mat_destroy": ([V], ctypes.c_int),
@@ -241,6 +242,10 @@ class Context:
     @property
     def stream(self) -> int:
         return int(_lib.hss_ctx_stream(self._h) or 0)
+
+    def trim(self):
+        """Free the device memory kept from destroyed factors and plans (``hss_ctx_trim``)."""
+        _check(_lib.hss_ctx_trim(self._h))
 
     def close(self):
         if self._h:

@@ -71,6 +71,8 @@ function Context(device::Integer=0)
     finalizer(c -> ccall((:hss_ctx_destroy, libhss), Cint, (Ptr{Cvoid},), c.h), c)
     return c
 end
+# frees the device memory kept from destroyed factors and plans
+trim(c::Context) = check(ccall((:hss_ctx_trim, libhss), Cint, (Ptr{Cvoid},), c.h))
 const DEFAULT_CTX = Ref{Union{Nothing,Context}}(nothing)
 default_context() = something(DEFAULT_CTX[], (DEFAULT_CTX[] = Context(0)))
 

@@ -108,6 +108,10 @@ typedef struct hss_solve_report {
 /* ---- context: owns the HIP stream used by every call on its handles ---- */
 hss_status hss_ctx_create(int device, hss_ctx_t* out);
 hss_status hss_ctx_destroy(hss_ctx_t ctx);
+/* Frees the device memory that the context keeps for its next factors, plans and host-pointer
+ * calls (at most 2 GiB, from ones destroyed before).  The library does so by itself when an
+ * allocation of its own fails; this is for memory that others are about to allocate. */
+hss_status hss_ctx_trim(hss_ctx_t ctx);
 /* hipStream_t of the context, for callers that enqueue around hss_*_dev calls */
 void* hss_ctx_stream(hss_ctx_t ctx);
 
