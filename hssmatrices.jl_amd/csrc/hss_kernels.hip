@@ -2754,40 +2754,46 @@ __global__ __launch_bounds__(256) void k_resid_norms(const double* __restrict__ 
 
 // Batched refinement helpers: block (request, column).
 // r = b - r (r holds A x on entry); norms[2*(req*maxc + col)] = ||b||^2, [+1] = ||r||^2.
-// Latency-bound where requests are few: 1024 threads with four rows each in flight take a
+// Four rows of a thread in flight.  Latency-bound where requests are few: 1024 threads take a
 // 32768-row column in 8 rounds (256 threads, one row at a time, were 128 rounds and 64 us
-// for 16 requests of up to 32 columns; now 32 us).
-__global__ __launch_bounds__(1024) void k_resid_batch(const BatchVec* __restrict__ tab, int maxc, double* __restrict__ norms) {
+// for 16 requests of up to 32 columns; now 32 us).  Columns of up to BATCH_WIDE_ROWS rows on
+// average run 256 threads: short of rows, three of four of 1024 threads wait at a quarter of the
+// workgroups a CU (256 requests of 400 rows: 29 us, 14 with 256 threads, 15 with one row at a
+// time; of 1000 rows 24, 17 and 19; 128 of 2000 rows 18.5, 16.7 and 19; 64 of 4000 24.5, 26.6 and 25).
+constexpr int64_t BATCH_WIDE_ROWS = 2048;
+template <int NT>
+__global__ __launch_bounds__(NT) void k_resid_batch(const BatchVec* __restrict__ tab, int maxc, double* __restrict__ norms) {
     const BatchVec v = tab[blockIdx.x];
     const int j = blockIdx.y;
     if (j >= v.nrhs) return;
     double nb, nr;
-    resid_norms<1024, 4>(v.b + j * v.ldb, v.r + j * v.n, 0, v.n, nb, nr);
+    resid_norms<NT, 4>(v.b + j * v.ldb, v.r + j * v.n, 0, v.n, nb, nr);
     if (threadIdx.x == 0) {
         norms[2 * ((int64_t)blockIdx.x * maxc + j)] = nb;
         norms[2 * ((int64_t)blockIdx.x * maxc + j) + 1] = nr;
     }
 }
 
-// x += d for active requests, block (request, column), 1024 threads with four rows each in
-// flight as above (38 -> 19 us)
-__global__ __launch_bounds__(1024) void k_axpy_batch(const BatchVec* __restrict__ tab) {
+// x += d for active requests, block (request, column), four rows of a thread in flight as
+// above (38 -> 19 us)
+template <int NT>
+__global__ __launch_bounds__(NT) void k_axpy_batch(const BatchVec* __restrict__ tab) {
     const BatchVec v = tab[blockIdx.x];
     const int j = blockIdx.y;
     if (j >= v.nrhs) return;
     double* __restrict__ x = v.x + j * v.ldx;
     const double* __restrict__ d = v.d + j * v.n;
-    for (int64_t i = threadIdx.x; i < v.n; i += 4 * 1024) {
+    for (int64_t i = threadIdx.x; i < v.n; i += 4 * NT) {
         double xv[4], dv[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int64_t e = i + q * 1024;
+            const int64_t e = i + q * NT;
             xv[q] = e < v.n ? x[e] : 0.0;
             dv[q] = e < v.n ? d[e] : 0.0;
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            if (i + q * 1024 < v.n) x[i + q * 1024] = xv[q] + dv[q];
+            if (i + q * NT < v.n) x[i + q * NT] = xv[q] + dv[q];
     }
 }
 
@@ -3075,14 +3081,16 @@ hipError_t launch_refine_check(BatchVec* tab, char* sinst0, char* sinst1, int64_
             norms, tol, rel, out);
     return hipGetLastError();
 }
-hipError_t launch_resid_batch(const BatchVec* tab, int cnt, int maxc, double* norms, hipStream_t st) {
+hipError_t launch_resid_batch(const BatchVec* tab, int cnt, int maxc, int64_t mean_rows, double* norms, hipStream_t st) {
     if (cnt <= 0 || maxc <= 0) return hipSuccess;
-    klaunch(k_resid_batch, dim3(cnt, maxc), dim3(1024), 0, st, tab, maxc, norms);
+    if (mean_rows > BATCH_WIDE_ROWS) klaunch((k_resid_batch<1024>), dim3(cnt, maxc), dim3(1024), 0, st, tab, maxc, norms);
+    else klaunch((k_resid_batch<256>), dim3(cnt, maxc), dim3(256), 0, st, tab, maxc, norms);
     return hipGetLastError();
 }
-hipError_t launch_axpy_batch(const BatchVec* tab, int cnt, int maxc, hipStream_t st) {
+hipError_t launch_axpy_batch(const BatchVec* tab, int cnt, int maxc, int64_t mean_rows, hipStream_t st) {
     if (cnt <= 0 || maxc <= 0) return hipSuccess;
-    klaunch(k_axpy_batch, dim3(cnt, maxc), dim3(1024), 0, st, tab);
+    if (mean_rows > BATCH_WIDE_ROWS) klaunch((k_axpy_batch<1024>), dim3(cnt, maxc), dim3(1024), 0, st, tab);
+    else klaunch((k_axpy_batch<256>), dim3(cnt, maxc), dim3(256), 0, st, tab);
     return hipGetLastError();
 }
 

@@ -97,8 +97,9 @@ hipError_t launch_gemm_tasks(const GemmTask* tasks, int count, hipStream_t st);
 hipError_t launch_refine_check(BatchVec* tab, char* sinst0, char* sinst1, int64_t sinst_size, int nrhs_off,
                                MvInst* mv, int cnt, int maxc, const double* norms, double tol, double* rel, int* out,
                                hipStream_t st);
-hipError_t launch_resid_batch(const BatchVec* tab, int cnt, int maxc, double* norms, hipStream_t st);
-hipError_t launch_axpy_batch(const BatchVec* tab, int cnt, int maxc, hipStream_t st);
+// mean_rows = rows of a column of the batch, on average
+hipError_t launch_resid_batch(const BatchVec* tab, int cnt, int maxc, int64_t mean_rows, double* norms, hipStream_t st);
+hipError_t launch_axpy_batch(const BatchVec* tab, int cnt, int maxc, int64_t mean_rows, hipStream_t st);
 hipError_t launch_residual(const double* B, int64_t ldb, double* R, int64_t ldr, int64_t n, int nrhs, hipStream_t st);
 // rows of one workgroup of launch_resid_norms; out holds 2 nrhs ceil(n / RESID_ROWS) values
 constexpr int RESID_ROWS = 4096;

@@ -2839,6 +2839,8 @@ struct hss_plan_s {
     bool holds_refs = false;  // false for the plans a factor caches for itself
     hss_prec prec = HSS_PREC_FP64;
     int cnt = 0, maxnrhs = 0;
+    int64_t cols = 0, colrows = 0;  // columns of all requests, their rows in all
+    int64_t mean_rows() const { return colrows / std::max<int64_t>(cols, 1); }
     bool has_ir = false;
     std::vector<SolveReq> reqs;
     char* arena = nullptr;
@@ -3011,6 +3013,8 @@ static hss_status plan_create_impl(int32_t count, hss_fact_s* const* facts, cons
         }
         P->reqs.push_back(SolveReq{F, nrhs[i], dB[i], ldb[i], dX[i], ldx[i]});
         P->maxnrhs = std::max(P->maxnrhs, (int)nrhs[i]);
+        P->cols += nrhs[i];
+        P->colrows += (int64_t)F->mat->rows * nrhs[i];
         P->lgroot = std::max(P->lgroot, F->lds_groot);
         P->lgroot_res = std::max(P->lgroot_res, F->lds_groot_res);
         P->lgroot2 = std::max(P->lgroot2, F->lds_groot2);
@@ -3301,7 +3305,7 @@ extern "C" hss_status hss_plan_execute(hss_plan_t P, const hss_refine_opts* opts
     auto enqueue_check = [&](int slot) -> hss_status {
         hss_status c = plan_matvec(P);  // r = A x
         if (c != HSS_OK) return c;
-        HIP_TRY(launch_resid_batch(P->d_vec, P->cnt, P->maxnrhs, P->d_norms, st));
+        HIP_TRY(launch_resid_batch(P->d_vec, P->cnt, P->maxnrhs, P->mean_rows(), P->d_norms, st));
         HIP_TRY(launch_refine_check(P->d_vec, P->d_sinst[0], P->d_sinst[1], (int64_t)P->sinst_size, (int)nrhs_off,
                                     P->d_mv, P->cnt, P->maxnrhs, P->d_norms, opts->tol, P->d_rel,
                                     P->d_count + slot, st));
@@ -3311,7 +3315,7 @@ extern "C" hss_status hss_plan_execute(hss_plan_t P, const hss_refine_opts* opts
     auto enqueue_solve = [&]() -> hss_status {
         hss_status c = fp32 ? plan_solve<float>(P, 1) : plan_solve<double>(P, 1);  // d = A \ r
         if (c != HSS_OK) return c;
-        HIP_TRY(launch_axpy_batch(P->d_vec, P->cnt, P->maxnrhs, st));  // x += d
+        HIP_TRY(launch_axpy_batch(P->d_vec, P->cnt, P->maxnrhs, P->mean_rows(), st));  // x += d
         return HSS_OK;
     };
     const bool graphs = !g_prof;
@@ -3631,6 +3635,7 @@ static hss_status server_round(hss_server_s* S) {
     // 2. tables: solve (first solve b->x, or correction r->d), axpy, matvec x->r, residual
     size_t ws = 0;
     int maxnrhs = 0;
+    int64_t cols = 0, colrows = 0;  // columns of all requests, their rows in all
     size_t lgroot = 0, lgroot_res = 0, lgroot2 = 0, lgroot2s = 0;
     bool all_groot2 = true;
     std::vector<size_t> off_s(cnt), off_m(cnt);
@@ -3645,6 +3650,8 @@ static hss_status server_round(hss_server_s* S) {
         off_m[i] = ws;
         ws = align256(ws + sizeof(double) * (size_t)(M->zrows + M->frows) * q->nrhs);
         maxnrhs = std::max(maxnrhs, q->nrhs);
+        cols += q->nrhs;
+        colrows += (int64_t)M->rows * q->nrhs;
         lgroot = std::max(lgroot, F->lds_groot);
         lgroot_res = std::max(lgroot_res, F->lds_groot_res);
         lgroot2 = std::max(lgroot2, F->lds_groot2);
@@ -3720,14 +3727,14 @@ static hss_status server_round(hss_server_s* S) {
     // 3. one batched solve, the corrections, one batched matvec + residual
     s = launch_schedule<TF>(dsi, dr, sch, maxnrhs, lgroot, lgroot_res, all_groot2 ? lgroot2 : 0, lgroot2s, st);
     if (s != HSS_OK) return s;
-    HIP_TRY(launch_axpy_batch(dbv, cnt, maxnrhs, st));
+    HIP_TRY(launch_axpy_batch(dbv, cnt, maxnrhs, colrows / cols, st));
     s = launch_mv_schedule(dmv, dw, mvs, maxnrhs, st);
     if (s != HSS_OK) return s;
     // the residual pass needs every request active: rewrite nrhs of the BatchVec rows
     for (int i = 0; i < cnt; ++i) bv[i].nrhs = S->inflight[i]->nrhs;
     HIP_TRY(hipMemcpyAsync(S->d_tab + o_bv, bv.data(), sizeof(BatchVec) * cnt, hipMemcpyHostToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));  // bv must stay valid until the copy is done
-    HIP_TRY(launch_resid_batch(dbv, cnt, maxnrhs, S->d_norms, st));
+    HIP_TRY(launch_resid_batch(dbv, cnt, maxnrhs, colrows / cols, S->d_norms, st));
     std::vector<double> norms(2 * (size_t)cnt * maxnrhs);
     HIP_TRY(hipMemcpyAsync(norms.data(), S->d_norms, nb, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
