@@ -1248,9 +1248,15 @@ __global__ __launch_bounds__(256) void k_ulv_wy(const FInst<T>* __restrict__ ins
 // wave searches the pivot for itself, and a step has three barriers.  In memory, with four
 // barriers a step and the merge one output a thread, it took 132 us on the n = 65536 log kernel
 // (86 now), 69 us on the n = 2001 Cauchy matrix (50) and 104 us on 32 Cauchy matrices (71).
-constexpr int ROOT_THREADS = 512;
-template <typename T, bool L>
-__global__ __launch_bounds__(ROOT_THREADS) void k_ulv_root(const FInst<T>* __restrict__ insts,
+// A block that stays in memory: Float64 with 512 threads as long as the roots of an XCD share its
+// L2 (one root of 300 rows 4.0 ms, 4.35 with 1024, 4.6 as first written: four barriers, 1024
+// threads, one wave's search, the update element by element); Float32, and Float64 beyond the
+// L2, with 1024 (Float32 of 300 rows 2.05 ms, 3.3 with 512, 2.75 as first written; 64 Float64
+// roots of 400 rows 9.3, 13.6 and 10.2).  Where every CU has a root and they do not fit, the traffic
+// counts: E updates element by element, in whole lines, and one wave searches (256 Float64 roots
+// of 500 rows 39 ms, 62 with 512 threads, 43 with 1024 without E, 41 as first written).
+template <typename T, bool L, int NT, bool E>
+__global__ __launch_bounds__(NT) void k_ulv_root(const FInst<T>* __restrict__ insts,
                                                            const WorkItem* __restrict__ work) {
     const WorkItem wi = work[blockIdx.x];
     const FInst<T>& I = insts[wi.inst];
@@ -1302,7 +1308,7 @@ __global__ __launch_bounds__(ROOT_THREADS) void k_ulv_root(const FInst<T>* __res
         // i, so an all-NaN column pivots in range (and is reported below)
         T best = T(-1);
         int p = i;
-        for (int rr = i + lane; rr < m; rr += 64) {
+        for (int rr = i + lane; rr < m && (!E || wave == 0); rr += 64) {
             const T v = fabs(A[rr + i * lda]);
             if (v > best) { best = v; p = rr; }
         }
@@ -1310,6 +1316,12 @@ __global__ __launch_bounds__(ROOT_THREADS) void k_ulv_root(const FInst<T>* __res
             const T ob = __shfl_xor(best, o, 64);
             const int oi = __shfl_xor(p, o, 64);
             if (ob > best || (ob == best && oi < p)) { best = ob; p = oi; }
+        }
+        if constexpr (E) {
+            __shared__ int s_p;
+            if (tid == 0) s_p = p;
+            __syncthreads();
+            p = s_p;
         }
         const T pv = A[p + i * lda];
         if (tid == 0) piv[i] = p;
@@ -1338,9 +1350,17 @@ __global__ __launch_bounds__(ROOT_THREADS) void k_ulv_root(const FInst<T>* __res
             A[rr + i * lda] = v * rcp;
         }
         __syncthreads();
-        for (int rr = i + 1 + lane; rr < m; rr += 64) {
-            const T l = A[rr + i * lda];
-            for (int c = i + 1 + wave; c < m; c += ROOT_THREADS / 64) A[rr + c * lda] -= l * A[i + c * lda];
+        if constexpr (E) {
+            const int mm = m - i - 1;
+            for (int e = tid; e < mm * mm; e += NT) {
+                const int rr = i + 1 + e % mm, c = i + 1 + e / mm;
+                A[rr + c * lda] -= A[rr + i * lda] * A[i + c * lda];
+            }
+        } else {
+            for (int rr = i + 1 + lane; rr < m; rr += 64) {
+                const T l = A[rr + i * lda];
+                for (int c = i + 1 + wave; c < m; c += NT / 64) A[rr + c * lda] -= l * A[i + c * lda];
+            }
         }
         __syncthreads();
     }
@@ -2867,13 +2887,17 @@ hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwor
     if (nwork <= 0) return hipSuccess;
     const size_t lds = sizeof(T) * (size_t)max_m * (size_t)(max_m | 1);
     if (lds <= 160 * 1024) {
-        const void* fn = reinterpret_cast<const void*>(&k_ulv_root<T, true>);
+        const void* fn = reinterpret_cast<const void*>(&k_ulv_root<T, true, 512, false>);
         hipError_t e = set_lds_attr<T>(fn, lds);
         if (e != hipSuccess) return e;
-        klaunch((k_ulv_root<T, true>), dim3(nwork), dim3(ROOT_THREADS), lds, st, insts, work);
-    } else {
-        klaunch((k_ulv_root<T, false>), dim3(nwork), dim3(ROOT_THREADS), 0, st, insts, work);
+        klaunch((k_ulv_root<T, true, 512, false>), dim3(nwork), dim3(512), lds, st, insts, work);
+        return hipGetLastError();
     }
+    // in memory, by whether the blocks of the roots that share an XCD fit its 4 MB L2
+    const bool fits = (size_t)((nwork + 7) / 8) * max_m * max_m * sizeof(T) <= size_t(4) << 20;
+    if (fits && sizeof(T) == 8) klaunch((k_ulv_root<T, false, 512, false>), dim3(nwork), dim3(512), 0, st, insts, work);
+    else if (fits || nwork <= 128) klaunch((k_ulv_root<T, false, 1024, false>), dim3(nwork), dim3(1024), 0, st, insts, work);
+    else klaunch((k_ulv_root<T, false, 1024, true>), dim3(nwork), dim3(1024), 0, st, insts, work);
     return hipGetLastError();
 }
 template <typename T>
