@@ -559,7 +559,7 @@ __device__ __forceinline__ bool ulv_front(const FInst<T>& I, const DevNode& nd, 
     // after the barrier, while the others work on column jj - 1.  The chain of k reductions
     // and barriers bounds it (0.75 us a reflector with two barriers and one wave's norm).
     {
-        constexpr int XR = 4, CW = 4;  // rows of a lane (m <= 256), columns of a wave at once
+        constexpr int XR = 4, CW = 4;  // rows of a lane (256 in all; the host takes m <= 128), columns of a wave at once
         for (int jj = k - 1; jj >= 0; --jj) {
             const int p = m - k + jj;
             T* col = Us + (int64_t)jj * m;
@@ -1032,13 +1032,15 @@ __device__ __forceinline__ void lq_panels(typename Mfma<T>::v4 (&a)[NTILE], cons
 //   LQ of the first nk rows in panels of 16 reflectors (ulvfactor.jl:44,47,50): the panel's
 //   wave factors its own rows (dlarfg reflectors, each applied to the panel's later rows;
 //   cross-lane shuffles, no workgroup barrier), writes the reflectors V (16 x n) to LDS and
-//   forms their compact-WY T (dlarft forward, from the Gram V V' on MFMA); then every wave
+//   forms their compact-WY T (dlarft forward, from the dots of the same steps); then every wave
 //   below applies the block, W <- W (I - V' T V) = W - ((W V') T) V, as three MFMA chains.
 //   One workgroup barrier per panel (V and T double-buffered).
 // Outputs as k_ulv_factor (L1, the LQ reflectors, L2a, V_top, the reduced D and V)
 // plus the T blocks and the inverted diagonal blocks of L1 (k_ulv_wy's outputs).
 // NTILE = 4 is held to four waves per SIMD, so that two workgroups share a CU on the batched
-// levels (one costs them 30 %).
+// levels (one costs them 30 %).  Its price in Float64: 179 registers spilled, in the panels'
+// reflector loop among others.  The eight-tile builds spill 32 (512 threads) and 356 (768
+// threads, the leaves of 128 rows).
 template <typename T, int NTILE, int NT>
 __global__ __launch_bounds__(NT, NT == 512 && NTILE == 4 ? 4 : 1) void k_ulv_factor_mf(const FInst<T>* __restrict__ insts,
                                                       const WorkItem* __restrict__ work) {
@@ -2758,7 +2760,7 @@ __device__ __forceinline__ void resid_norms(const double* __restrict__ b, double
 // Residual of one solve, block (column, chunk of RESID_ROWS rows): out[2 (chunk nrhs + j)] =
 // the chunk's share of ||b_j||^2, [+1] of ||r_j||^2; the host adds the chunks in order.
 // Bound by memory: two reads and a write.  One workgroup a column (as one norm of it was
-// before) is bound by latency instead, 64 us a norm of 65536 x 128; with 16 rows a thread in
+// before) is bound by latency instead, 64 us a norm of 65536 x 128; with 8 rows a thread in
 // flight and 16 x 128 workgroups the whole pass takes 32 us (residual and two norms: 160).
 __global__ __launch_bounds__(256) void k_resid_norms(const double* __restrict__ B, int64_t ldb, double* __restrict__ Rr,
                                                      int64_t ldr, int64_t n, int nrhs, double* __restrict__ out) {

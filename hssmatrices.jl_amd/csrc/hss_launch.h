@@ -47,9 +47,9 @@ template <typename T>
 hipError_t launch_ulv_wy(const FInst<T>* insts, const WorkItem* work, int nwork, hipStream_t st);
 template <typename T>
 hipError_t launch_ulv_root(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, hipStream_t st);
-// solve operators, once per factorization (every non-root node in one launch)
-// Gz, Gr and Qt of nodes with at most 128 rows (k_ulv_gform, k_ulv_qform); the factor kernels
-// take no larger ones: m S <= FACT_THREADS, and S = 8 from n = 129 on
+// solve operators, once per factorization: Gz, Gr and Qt of nodes with at most 128 rows, a launch
+// each (k_ulv_gform, k_ulv_qform) with the build for up to 64 rows or for 128.  The factor kernels
+// take no larger nodes: m S <= FACT_THREADS, and S = 8 from n = 129 on
 template <typename T>
 hipError_t launch_ulv_forms(const FInst<T>* insts, const WorkItem* work, int nwork, int max_m, int max_kx, int max_n,
                               hipStream_t st);

@@ -1939,7 +1939,7 @@ static hss_status plan_factor(hss_mat_s* M, hss_fact_s* F) {
         F->lds_groot2s = sizeof(TF) * (size_t)((2 * (int64_t)fr.m * fr.m + (int64_t)fr.m * fr.Kx + 15) / 16 * 16 + io);
     }
     if (most * tv > 160 * 1024 || F->lds_groot > 160 * 1024)
-        return fail(HSS_ERR_UNSUPPORTED, "a node exceeds the LDS of the solve-operator kernels");
+        return fail(HSS_ERR_UNSUPPORTED, "a node exceeds the size that the solve operators are formed for");
     return HSS_OK;
 }
 
@@ -2064,10 +2064,13 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
         lev_lds_mf[h] = std::max(lev_lds_mf[h], lev_lds[h]);
     }
     // Float64 levels run the blocked MFMA kernel when their nodes have n <= 128 and at most
-    // factor_mf_max_rows rows of [D; V'] (others run the per-reflector kernel).  Float32
-    // levels run the per-reflector kernel: measured on the n = 65536 log-kernel matrix
-    // (leaf 128, ranks 11-35), the blocked kernel is 10 % faster per level in Float64 and
-    // 0-20 % slower in Float32, whose per-reflector steps are cheaper.
+    // factor_mf_max_rows rows of [D; V'] (others run the per-reflector kernel): kernels of the
+    // whole factor 2175 us against 3424 (n = 65536 log, leaf 128), 487 against 902 (n = 2001
+    // Cauchy), 2680 against 6017 (32 Cauchy matrices).  Float32 levels run the per-reflector
+    // kernel.  That line was drawn when the blocked one was up to 20 % slower in Float32; as it is
+    // now it takes 1627 us against 2435, 379 against 674 and 1875 against 4150, but how many
+    // refinement steps its factors need on batches, which decided it then, has not been measured
+    // again.
     auto use_mf = [&](int h) {
         const bool want = g_factor_kernel == FactorKernel::Auto ? sizeof(TF) == 8 : g_factor_kernel == FactorKernel::Mfma;
         return want && lev_n[h] <= 128 && lev_rows[h] <= factor_mf_max_rows((int)sizeof(TF)) &&
@@ -2166,7 +2169,7 @@ static hss_status factor_batch(const std::vector<hss_mat_s*>& mats, hss_prec pre
             ProfScope ps("k_ulv_rinv", 0, roots.count, st);
             HIP_TRY((launch_ulv_rinv<TF>(d_inst, d_work + roots.off, roots.count, max_rcols, lds_rinv, st)));
         }
-        // solve operators G and Qt of every non-root node (one launch each)
+        // solve operators G and Qt of every non-root node (one launch each and size class)
         for (int c = 0; c < 2; ++c) {
             ProfScope ps("k_ulv_forms", c, form[c].r.count, st);
             HIP_TRY((launch_ulv_forms<TF>(d_inst, d_work + form[c].r.off, form[c].r.count, form[c].m, form[c].kx,
