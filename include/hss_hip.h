@@ -43,7 +43,7 @@ typedef enum hss_status {
     HSS_ERR_DIM = 1,      /* DimensionMismatch */
     HSS_ERR_ARG = 2,      /* ArgumentError / malformed tree */
     HSS_ERR_SINGULAR = 3, /* SingularException (zero pivot in the dense root solve) */
-    HSS_ERR_NOCONV = 4,   /* iterative refinement did not reach the requested residual */
+    HSS_ERR_NOCONV = 4,   /* iterative refinement did not reach the requested residual (a NaN never does) */
     HSS_ERR_OOM = 5,      /* device allocation failed */
     HSS_ERR_BUDGET = 6,   /* admission refused: over the memory budget */
     HSS_ERR_HIP = 7,      /* HIP runtime error */
